@@ -181,6 +181,10 @@ struct xme_plan {
     FsTask *d_tasks = nullptr;
     FsItem *d_items = nullptr;
     int32_t *d_item_insts = nullptr;
+    ElItem *d_el_items = nullptr;      // successive-elimination plans: the items instead of the two above
+    bool elim = false;
+    int el_threads = 0;                // workgroup size of the elimination search
+    bool el_few = false;               // fewer than 4 tasks per CU (xme_el_rows)
     int32_t *d_sp_list = nullptr;      // sub-pel PU order: small PUs, then large ones
     int n_sp_small = 0, n_sp_large = 0;
     uint32_t *d_counters = nullptr;
@@ -394,6 +398,106 @@ static std::vector<std::vector<int>> make_groups(const std::vector<DevPu> &pus, 
     return out;
 }
 
+// Candidate rows [row0, row0 + nrows) and all 2R columns of one PU around
+// centre (cx, cy): the window bytes the elimination search reads for them
+// (a lane's K rows stay inside the range when it has as many).
+static Rect el_footprint(const DevParams &p, const DevPu &pu, int row0, int nrows, int cx, int cy)
+{
+    Rect r;
+    r.x0 = pu.x + cx - p.R;
+    r.x1 = r.x0 + 2 * p.R + pu.w - 1;
+    r.y0 = pu.y + cy - p.R + row0;
+    r.y1 = r.y0 + std::max(nrows, xme_el_rows(p.R, false, pu.w, pu.h)) + pu.h - 1;
+    return r;
+}
+
+// A task of the elimination search over candidate rows [row_lo, row_hi) of
+// the given PUs against one reference; item_begin / item_end are the caller's.
+// Returns its LDS bytes apart from the waves' areas.
+static size_t el_task(const DevParams &p, const std::vector<DevPu> &pus, const std::vector<int> &members, int ref,
+                      int row_lo, int row_hi, FsTask &t)
+{
+    Rect win = { 1 << 30, 1 << 30, -(1 << 30), -(1 << 30) };
+    Rect cur = win;
+    for (int i : members) {
+        const DevPu &pu = pus[i];
+        int c[2][2];
+        const int n = possible_centres(p, pu, c);
+        for (int k = 0; k < n; k++)
+            win.add(el_footprint(p, pu, row_lo, row_hi - row_lo, c[k][0], c[k][1]));
+        cur.add(Rect{ pu.x, pu.y, pu.x + pu.w, pu.y + pu.h });
+    }
+    t.ref = ref;
+    const int wx0 = (int)std::floor(win.x0 / 4.0) * 4;
+    t.wx0 = (int16_t)wx0;
+    t.wy0 = (int16_t)win.y0;
+    t.ww = (int16_t)(((win.x1 - wx0) + 3) & ~3);
+    t.wh = (int16_t)(win.y1 - win.y0);
+    t.cx0 = (int16_t)cur.x0;
+    t.cy0 = (int16_t)cur.y0;
+    t.cw = (int16_t)(((cur.x1 - cur.x0) + 3) & ~3);
+    t.ch = (int16_t)(cur.y1 - cur.y0);
+    return ((size_t)xme_el_pitch(t.ww) * t.wh + (size_t)(t.cw >> 2) * t.ch +
+            (size_t)xme_el_sum_pitch(t.ww) * (t.wh - 3)) * 4 + 16;
+}
+
+// The tasks of an elimination search, for every reference, before they are
+// filled: PUs and candidate rows [lo, hi).
+struct ElCut {
+    std::vector<int> members;
+    int lo, hi;
+    FsTask task;
+};
+
+// Cuts the PUs of one cell of the picture (a square of 1 << level) into tasks
+// of at most `cap` bytes of window, sums and pixels: the candidate rows in two
+// at most, else the cell in quarters (a group's search centres spread less),
+// and a PU that is alone in as many row ranges as it takes.  False when even
+// K rows of one PU (whose window spans both its possible centres) do not fit,
+// or when anything has to be cut and `whole` asks for none of it.
+static bool el_cuts(const DevParams &p, const std::vector<DevPu> &pus, const std::vector<int> &members, int level,
+                    size_t cap, bool whole, std::vector<ElCut> &out, size_t &staged)
+{
+    const int K = xme_el_rows(p.R, false, 4, 4), R2 = 2 * p.R;      // the most any PU takes
+    for (int splits = 1; splits <= 2 || members.size() == 1; splits *= 2) {
+        const int per = std::max(K, (R2 + splits - 1) / splits);
+        const size_t before = out.size();
+        size_t need = 0;
+        for (int lo = 0; lo < R2 && need <= cap; lo += per) {
+            ElCut c{ {}, lo, std::min(R2, lo + per), {} };
+            need = std::max(need, el_task(p, pus, members, 0, c.lo, c.hi, c.task));
+            c.members = members;
+            out.push_back(std::move(c));
+        }
+        if (need <= cap) {
+            staged = std::max(staged, need);
+            return true;
+        }
+        out.resize(before);
+        if (whole || (per == K && members.size() == 1))
+            return false;
+    }
+    std::map<std::pair<int, int>, std::vector<int>> cells;
+    if (level > 3)
+        for (int i : members)
+            cells[{ pus[i].y >> (level - 1), pus[i].x >> (level - 1) }].push_back(i);
+    else
+        for (int i : members)
+            cells[{ i, 0 }].push_back(i);
+    for (auto &kv : cells)
+        if (!el_cuts(p, pus, kv.second, level - 1, cap, false, out, staged))
+            return false;
+    return true;
+}
+
+// Relative time of an item: what a candidate costs in the bound (its
+// sub-blocks) and what its share of surviving tiles costs, with the
+// per-candidate overheads.
+static int64_t el_cost(const DevParams &p, const DevPu &pu, int nrows)
+{
+    return (int64_t)nrows * 2 * p.R * (8 + pu.w * pu.h / 10);
+}
+
 // Build a task from items of one reference.  Returns the LDS bytes it needs.
 static size_t make_task(const DevParams &p, const std::vector<DevPu> &pus, const std::vector<HostItem> &its,
                         int ref, FsTask &t)
@@ -424,6 +528,39 @@ static size_t make_task(const DevParams &p, const std::vector<DevPu> &pus, const
     return ((staged + 15) & ~(size_t)15) + XME_FS_TERM_BYTES;
 }
 
+// Whether the exhaustive search's windows of one CTU's PUs fit `cap` bytes of
+// LDS at its finest split in candidate rows (the limit that a batched plan is
+// refused at, whichever search takes it).
+static bool fs_windows_fit(const DevParams &p, const std::vector<DevPu> &pus, const std::vector<int> &members, size_t cap)
+{
+    const int R2 = 2 * p.R;
+    int splits = 1;
+    while (splits < R2 / 4)
+        splits *= 2;
+    const int rows_per = (R2 + splits - 1) / splits;
+    for (int pass = 0; pass < 2; pass++) {
+        std::vector<int> insts;
+        for (int i : members)
+            if (uses_narrow(p, pus[i].part) == (pass == 1))
+                insts.push_back(i * p.n_ref);
+        if (insts.empty())
+            continue;
+        const auto groups = make_groups(pus, insts, p.n_ref, XME_MAX_GROUP, [&](int part) {
+            int K, LC;
+            return band_shape(p, part, 0, rows_per, K, LC);
+        });
+        for (int s = 0; s < splits && s * rows_per < R2; s++) {
+            std::vector<HostItem> items;
+            for (const auto &g : groups)
+                items_for(p, pus, g, pus[g[0] / p.n_ref].part, s * rows_per, std::min(R2, (s + 1) * rows_per), items);
+            FsTask t;
+            if (!items.empty() && make_task(p, pus, items, 0, t) > cap)
+                return false;
+        }
+    }
+    return true;
+}
+
 } // namespace
 
 static void plan_free(xme_plan *pl)
@@ -438,6 +575,7 @@ static void plan_free(xme_plan *pl)
     hipFree(pl->d_tasks);
     hipFree(pl->d_items);
     hipFree(pl->d_item_insts);
+    hipFree(pl->d_el_items);
     hipFree(pl->d_sp_list);
     hipFree(pl->d_pat_list);
     hipFree(pl->d_pat_points);
@@ -636,6 +774,7 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
     std::vector<FsTask> tasks;
     std::vector<FsItem> items;
     std::vector<int32_t> item_insts;
+    std::vector<ElItem> el_items;
     std::vector<int> task_part;
     const int R2 = 2 * p.R;
 
@@ -661,6 +800,52 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
         return lds;
     };
 
+    // The successive-elimination search takes the batched full searches whose
+    // columns one band of lanes spans (2 R <= 128) and whose windows fit the
+    // LDS with their sums; the others, plain plans and the tuner (which times
+    // the exhaustive tiles) search exhaustively.
+    std::vector<ElCut> cuts;
+    if (p.method == XME_ME_FS && mode == XME_PLAN_BATCHED && p.R <= XME_EL_MAX_R && !xme_tune_forced()) {
+        // one task per 64x64 CTU and reference (all PU shapes together); per
+        // quarter CTU when that gives fewer tasks than CUs (1080p 16x16 PUs,
+        // R = 32, 510 CTUs: 53 us whole, 85 us in quarters; 720p, R = 8, 240
+        // CTUs: 57 us in quarters)
+        const int level = ((p.frame_w + 63) / 64) * ((p.frame_h + 63) / 64) * n_ref < 256 ? 5 : 6;
+        auto grid = [&](int lv) {
+            const int gw = (p.frame_w >> lv) + 1;
+            std::vector<std::vector<int>> g((size_t)gw * ((p.frame_h >> lv) + 1));
+            for (int i = 0; i < n_pu; i++)
+                g[(size_t)(pus[i].y >> lv) * gw + (pus[i].x >> lv)].push_back(i);
+            g.erase(std::remove_if(g.begin(), g.end(), [](const std::vector<int> &m) { return m.empty(); }), g.end());
+            return g;
+        };
+        const auto ctus = grid(6);
+        const auto cells = level == 6 ? ctus : grid(level);
+        // a CTU's exhaustive window is a few columns and rows wider than el_task's
+        bool fit = true;
+        for (const auto &m : ctus) {
+            FsTask t;
+            el_task(p, pus, m, 0, 0, R2, t);
+            const size_t bytes = (size_t)(t.ww + 20) * (t.wh + 16) + (size_t)t.cw * t.ch + XME_FS_TERM_BYTES + 64;
+            fit = fit && (bytes <= lds_cap || fs_windows_fit(p, pus, m, lds_cap));
+        }
+        // 8 waves a workgroup when two such share a CU's LDS with whole windows, else 16
+        for (int waves : { 8, 16 }) {
+            const size_t areas = (size_t)waves * XME_EL_WAVE_BYTES;
+            const size_t cap = (waves == 8 ? lds_cap / 2 : lds_cap) - areas;
+            size_t staged = 0;
+            cuts.clear();
+            pl->elim = fit;        // else refused below, as ever
+            for (const auto &m : cells)
+                pl->elim = pl->elim && el_cuts(p, pus, m, level, cap, waves == 8, cuts, staged);
+            pl->el_threads = 64 * waves;
+            pl->lds_bytes = staged + areas;
+            if (pl->elim)
+                break;
+        }
+        pl->el_few = cuts.size() * n_ref < 1024;
+    }
+
     std::vector<int32_t> pat_list;
     if (p.method != XME_ME_FS) {
         // pattern searches: one launch in either mode, the instances of each
@@ -683,6 +868,55 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
             waves += nw;
             pl->pat_wave_end[k] = waves;
         }
+    } else if (pl->elim) {
+        std::vector<std::pair<int64_t, ElItem>> list;
+        for (const ElCut &c : cuts) {
+            // an item is the bands of a PU that make about the work of the
+            // full range of an 8x8 PU, so that a task's waves end together
+            for (int pass = 0; pass < 2; pass++) {
+                list.clear();
+                for (int i : c.members) {
+                    const DevPu &q = pus[i];
+                    const int K = xme_el_rows(p.R, pl->el_few, q.w, q.h), band = (64 >> xme_el_lc_log2(p.R)) * K;
+                    const int bands = pass ? 1 : std::max(1, 1024 * 16 / (q.w * q.h * K));
+                    for (int lo = c.lo, n; lo < c.hi; lo += n) {
+                        n = std::min(c.hi - lo, bands * band);
+                        if (c.hi - lo - n < K)
+                            n = c.hi - lo;          // no item of fewer than K rows
+                        list.push_back({ -el_cost(p, q, n), ElItem{ i * n_ref, (uint8_t)lo, (uint8_t)n, q.w, q.h, q.x, q.y,
+                                                                    q.mvp_x, q.mvp_y } });
+                    }
+                }
+                if ((int)list.size() >= pl->el_threads / 64)
+                    break;
+            }
+            std::stable_sort(list.begin(), list.end(), [](const auto &a, const auto &b) { return a.first < b.first; });
+            for (int r = 0; r < n_ref; r++) {
+                FsTask t = c.task;
+                t.ref = r;
+                t.item_begin = (int)el_items.size();
+                for (const auto &e : list) {
+                    el_items.push_back(e.second);
+                    el_items.back().inst += r;
+                }
+                t.item_end = (int)el_items.size();
+                tasks.push_back(t);
+            }
+        }
+        auto work = [&](const FsTask &t) {
+            int64_t w = 0;
+            for (int k = t.item_begin; k < t.item_end; k++)
+                w += el_cost(p, pus[el_items[k].inst / n_ref], el_items[k].nrows);
+            return w;
+        };
+        std::vector<std::pair<int64_t, int>> order(tasks.size());
+        for (size_t k = 0; k < tasks.size(); k++)
+            order[k] = { -work(tasks[k]), (int)k };
+        std::sort(order.begin(), order.end());
+        std::vector<FsTask> sorted(tasks.size());
+        for (size_t k = 0; k < tasks.size(); k++)
+            sorted[k] = tasks[order[k].second];
+        tasks.swap(sorted);
     } else if (mode == XME_PLAN_BATCHED) {
         // group PUs by 64x64 CTU; split the candidate rows until the window fits.
         // Pass 0 builds the generic tasks, pass 1 the narrow-PU tasks.
@@ -787,6 +1021,11 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
     for (size_t ti = 0; ti < tasks.size(); ti++) {
         int64_t w = 0;
         for (int k = tasks[ti].item_begin; k < tasks[ti].item_end; k++) {
+            if (pl->elim) {
+                const DevPu &pu = pus[el_items[k].inst / n_ref];
+                w += (int64_t)pu.w * pu.h * el_items[k].nrows * R2;
+                continue;
+            }
             const FsItem &it = items[k];
             const DevPu &pu = pus[item_insts[it.list] / n_ref];
             w += (int64_t)it.count * pu.w * pu.h * it.nrows * it.ncols;
@@ -796,6 +1035,8 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
     split_launches(pl, 0);
 
     for (const FsTask &t : tasks) {
+        if (pl->elim)
+            break;                 // sized above
         size_t need = (((size_t)window_pitch_host(t.ww) * t.wh + (size_t)t.cw * t.ch + 15) & ~(size_t)15) +
                       XME_FS_TERM_BYTES;
         if (need > lds_cap) {
@@ -817,6 +1058,7 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
     up((void **)&pl->d_tasks, tasks.data(), tasks.size() * sizeof(FsTask));
     up((void **)&pl->d_items, items.data(), items.size() * sizeof(FsItem));
     up((void **)&pl->d_item_insts, item_insts.data(), item_insts.size() * sizeof(int32_t));
+    up((void **)&pl->d_el_items, el_items.data(), el_items.size() * sizeof(ElItem));
     up((void **)&pl->d_pat_list, pat_list.data(), pat_list.size() * sizeof(int32_t));
     if (e == hipSuccess && p.method != XME_ME_FS) {
         e = plan_dev_alloc(pl, (void **)&pl->d_pat_points, sizeof(uint32_t) * pl->n_inst);
@@ -883,7 +1125,7 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
         return rc;
     }
     if (mode == XME_PLAN_BATCHED && p.method == XME_ME_FS) {
-        int prc = xme_fs_prepare();
+        int prc = pl->elim ? xme_el_prepare() : xme_fs_prepare();
         if (prc) {
             plan_free(pl);
             return prc;
@@ -892,8 +1134,10 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, pl->device);
         auto fill = [&](int variant, size_t lds, int n) {
             int per_cu = 0;
-            hipError_t oe = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, xme_fs_kernel_ptr(true, variant),
-                                                                          256, lds);
+            hipError_t oe = pl->elim ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, xme_el_kernel_ptr(p.R, pl->el_few),
+                                                                                    pl->el_threads, lds)
+                                     : hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                                           &per_cu, xme_fs_kernel_ptr(true, variant), 256, lds);
             if (oe != hipSuccess || per_cu < 1)
                 per_cu = 1;
             return std::max(1, std::min(per_cu * cus, n));
@@ -1091,6 +1335,14 @@ static int launch_search(xme_plan *pl, hipStream_t s)
         // launches of one variant run in stream order and share its queue
         // counters (the last workgroup of a launch resets them)
         for (const auto &c : pl->chunks_gen) {
+            if (pl->elim) {
+                rc = xme_launch_elim(pl->p, pl->d_desc, pl->d_inst, pl->d_tasks + c.first, c.second,
+                                     pl->d_el_items, pl->d_best, pl->d_counters, pl->lds_bytes,
+                                     std::min(pl->grid, c.second), pl->el_threads, pl->el_few, s);
+                if (rc)
+                    return rc;
+                continue;
+            }
             rc = xme_launch_fs(pl->p, pl->d_desc, pl->d_pus, pl->d_inst, pl->d_tasks + c.first, c.second, pl->d_items,
                                pl->d_item_insts, pl->d_best, pl->d_counters, pl->lds_bytes,
                                std::min(pl->grid, c.second), true, pl->kmax, s);
@@ -1141,7 +1393,10 @@ extern "C" int xme_me_run(xme_plan *pl, const pel_t *cur, intptr_t i_cur, const 
     int rc = fill_desc(pl, cur, i_cur, refs, res, cost_map, s);
     if (rc)
         return rc;
-    return launch_all(pl, s);
+    rc = launch_all(pl, s);
+    if (rc == XME_OK && cost_map && pl->elim)      // the elimination search does not cost every candidate
+        rc = xme_launch_cost_map(pl->p, pl->d_desc, pl->d_pus, pl->d_inst, pl->n_inst, s);
+    return rc;
 }
 
 extern "C" int xme_me_run_graph(xme_plan *pl, const pel_t *cur, intptr_t i_cur, const xme_ref_desc *refs,

@@ -94,6 +94,12 @@ void xme_tune_force(const TuneChoice *c)
     }
 }
 
+bool xme_tune_forced(void)
+{
+    std::lock_guard<std::mutex> lk(g_mu);
+    return g_forced;
+}
+
 extern "C" int xme_tune_get(int part, int R, int *k_rows, int *lanes_per_row)
 {
     if (part < 0 || part >= XME_NUM_PU)

@@ -13,6 +13,7 @@ TuneChoice xme_tune_default(int part, int search_range);
 void xme_tune_store(int part, int search_range, TuneChoice c);
 // Forces a choice for every shape (used by the tuner while it measures).
 void xme_tune_force(const TuneChoice *c);
+bool xme_tune_forced(void);
 
 int xme_part_index(int w, int h);
 // At most 256 pixels (every shape up to 16 x 16, 8 x 32 and 32 x 8):

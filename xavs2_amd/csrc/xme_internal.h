@@ -75,6 +75,16 @@ struct FsItem {
     uint8_t K, LC;             // rows per lane, lanes per candidate row
     uint8_t pad[2];
 };
+// A wave work item of the successive-elimination search: candidate rows
+// [row0, row0 + nrows) of one (PU, reference) instance, with its PU's fields.
+struct ElItem {
+    int32_t inst;
+    uint8_t row0, nrows;       // [0, 2 * XME_EL_MAX_R]
+    uint8_t w, h;
+    int16_t x, y;
+    int16_t mvp_x, mvp_y;
+};
+static_assert(sizeof(ElItem) == 16, "the search kernel moves an item as four dwords");
 // Instances of one item: one per lane when the search kernel fetches them.
 #define XME_MAX_GROUP 64
 static_assert(XME_MAX_GROUP <= 64, "an item's instances are fetched one per lane");
@@ -189,6 +199,25 @@ int xme_launch_fs(const DevParams &p, const FrameDesc *d_desc, const DevPu *d_pu
 // LDS bytes of a search task beyond its staged window and current pixels
 // (per-wave MV-cost term tables of 4 waves x 8 x 4 x 64 dwords).
 #define XME_FS_TERM_BYTES (4 * 8 * 4 * 64 * 4)
+// The successive-elimination search (elim_kernels.hip): batched plans of
+// search ranges up to XME_EL_MAX_R.  LDS of a task: the window
+// (xme_el_pitch dwords a row), the current pixels, the window's 4x4 sums
+// (xme_el_sum_pitch dwords a row, 3 rows fewer), then XME_EL_WAVE_BYTES per
+// wave of the workgroup.
+#define XME_EL_MAX_R 64
+#define XME_EL_WAVE_BYTES 2688
+__host__ __device__ inline int xme_el_pitch(int ww) { return (ww >> 2) | 1; }
+__host__ __device__ inline int xme_el_sum_pitch(int ww) { return (ww >> 1) | 1; }
+int xme_el_rows(int R, bool few_tasks, int w, int h);     // candidate rows per lane for a w x h PU
+int xme_el_lc_log2(int R);     // log2 of the lanes per candidate row
+const void *xme_el_kernel_ptr(int R, bool few_tasks);
+int xme_el_prepare(void);
+int xme_launch_elim(const DevParams &p, const FrameDesc *d_desc, const DevInst *d_inst, const FsTask *d_tasks,
+                    int n_tasks, const ElItem *d_items, uint64_t *d_best, uint32_t *d_counters, size_t lds_bytes, int grid,
+                    int threads, bool few_tasks, hipStream_t s);
+// Raster costs of every candidate into the frame's cost map (diagnostics).
+int xme_launch_cost_map(const DevParams &p, const FrameDesc *d_desc, const DevPu *d_pus, const DevInst *d_inst,
+                        int n_inst, hipStream_t s);
 // Sub-pel refinement of every instance.  `d_list` holds PU indices: the
 // first n_small PUs have at most 64 4x4 tiles (xme_subpel_large false), the
 // next n_large more; each part gets a kernel variant of its own.
