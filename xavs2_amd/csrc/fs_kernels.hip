@@ -26,26 +26,18 @@
 namespace {
 
 // ---------------------------------------------------------------------------
-// Candidate-list pass: a group of 16 lanes per (PU, reference), four groups a
-// wave, 16 a workgroup; workgroup b runs on XCD b % 8, and the instances are
-// walked reference-major in contiguous ranges per XCD so that neighbouring
-// PUs of one reference share an L2.  A PU of more than 16 pixel quads loops
-// over them (the groups of a wave run their loops independently; the sums
-// follow once the wave has reconverged).
-__global__ void __launch_bounds__(256) mvc_kernel(DevParams p, const FrameDesc *__restrict__ desc,
-                                                  const DevPu *__restrict__ pus, DevInst *__restrict__ inst,
-                                                  uint64_t *__restrict__ best, int n_inst)
+// Candidate-list pass: 16 lanes per (PU, reference), or a workgroup of 256 for
+// PUs of more than 1024 pixels (sub-pel class 3: their 512 to 1024 dwords took
+// a group of 16 lanes 32 to 64 dependent reads, the whole kernel's time on a
+// small frame: 424x240 21.7 -> 5 us).  The large instances come first; the
+// others are walked reference-major in contiguous ranges per XCD (workgroup b
+// runs on XCD b % 8), so that neighbouring PUs of one reference share an L2.
+template <int S>
+__device__ __forceinline__ void mvc_instance(const DevParams &p, const FrameDesc *__restrict__ desc,
+                                             const DevPu *__restrict__ pus, DevInst *__restrict__ inst,
+                                             uint64_t *__restrict__ best, int pu_i, int r, bool live, int *part)
 {
-    constexpr int S = 16;
-    const int per_xcd = gridDim.x / 8;
-    const int lb = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    const int lane = threadIdx.x & 63, l = lane & (S - 1);
-    const int logical = lb * 16 + (int)(threadIdx.x >> 4);
-    if (__builtin_amdgcn_readfirstlane(lb * 16 + (int)((threadIdx.x >> 6) << 2)) >= n_inst)
-        return;   // the whole wave is past the end
-    const bool live = logical < n_inst;
-    const int li = live ? logical : 0;
-    const int r = li / p.n_pu, pu_i = li - r * p.n_pu;
+    const int l = threadIdx.x & (S - 1);
     const int id = pu_i * p.n_ref + r;
     const DevPu pu = pus[pu_i];
     const MvWindow win = xme_mv_window(p, pu.x, pu.y, pu.w, pu.h);
@@ -82,9 +74,11 @@ __global__ void __launch_bounds__(256) mvc_kernel(DevParams p, const FrameDesc *
         rp[c] = ref + (int64_t)(ok[c] ? cand[c][1] : 0) * i_ref + (ok[c] ? cand[c][0] : 0);
     }
     uint32_t sad[2] = { 0, 0 };
-    const int gw = pu.w >> 2;
-    for (int t = l; live && t < gw * pu.h; t += S) {
-        const int yy = t / gw, xx = (t - yy * gw) * 4;
+    const int gw = pu.w >> 2, total = live ? gw * pu.h : 0;
+    const uint32_t inv = 65536u / (uint32_t)gw + 1;      // t / gw for t < 1024, gw <= 16
+#pragma unroll 4
+    for (int t = l; t < total; t += S) {
+        const int yy = (int)(__umul24((uint32_t)t, inv) >> 16), xx = (t - yy * gw) * 4;
         const uint32_t c4 = *(gdwords)(cur + (int64_t)yy * desc->i_cur + xx);
 #pragma unroll
         for (int c = 0; c < 2; c++) {
@@ -99,7 +93,17 @@ __global__ void __launch_bounds__(256) mvc_kernel(DevParams p, const FrameDesc *
     int tot[2];
 #pragma unroll
     for (int c = 0; c < 2; c++)
-        tot[c] = group_sum((int)sad[c], S);
+        tot[c] = group_sum((int)sad[c], S < 64 ? S : 64);
+    if constexpr (S == 256) {
+        const int wave = threadIdx.x >> 6;
+        if ((threadIdx.x & 63) == 63) {
+            part[2 * wave] = tot[0];
+            part[2 * wave + 1] = tot[1];
+        }
+        __syncthreads();
+        tot[0] = part[0] + part[2] + part[4] + part[6];
+        tot[1] = part[1] + part[3] + part[5] + part[7];
+    }
     if (!live || l != S - 1)
         return;
     uint64_t key = XME_KEY_NONE;
@@ -129,6 +133,33 @@ __global__ void __launch_bounds__(256) mvc_kernel(DevParams p, const FrameDesc *
     d.flags = 0;
     inst[id] = d;
     best[id] = key;
+}
+
+__global__ void __launch_bounds__(256) mvc_kernel(DevParams p, const FrameDesc *__restrict__ desc,
+                                                  const DevPu *__restrict__ pus, DevInst *__restrict__ inst,
+                                                  uint64_t *__restrict__ best, const int32_t *__restrict__ list,
+                                                  int n_small, int n_large)
+{
+    __shared__ int s_part[8];
+    const int n_large_wg = n_large * p.n_ref, large_blocks = (n_large_wg + 7) / 8 * 8;
+    int b = (int)blockIdx.x;
+    if (b < large_blocks) {
+        if (b < n_large_wg) {
+            const int r = b / n_large;
+            mvc_instance<256>(p, desc, pus, inst, best, list[n_small + b - r * n_large], r, true, s_part);
+        }
+        return;
+    }
+    b -= large_blocks;                       // b % 8 is unchanged
+    const int per_xcd = ((int)gridDim.x - large_blocks) / 8;
+    const int lb = (b % 8) * per_xcd + b / 8;
+    const int logical = lb * 16 + (int)(threadIdx.x >> 4), n_inst = n_small * p.n_ref;
+    if (__builtin_amdgcn_readfirstlane(lb * 16 + (int)((threadIdx.x >> 6) << 2)) >= n_inst)
+        return;   // the whole wave is past the end
+    const bool live = logical < n_inst;
+    const int li = live ? logical : 0;
+    const int r = li / n_small;
+    mvc_instance<16>(p, desc, pus, inst, best, list[li - r * n_small], r, live, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1010,13 +1041,15 @@ int xme_fs_prepare(void)
 }
 
 int xme_launch_mvc(const DevParams &p, const FrameDesc *d_desc, const DevPu *d_pus, DevInst *d_inst,
-                   uint64_t *d_best, int n_inst, hipStream_t s)
+                   uint64_t *d_best, const int32_t *d_list, const SubpelCounts &n, hipStream_t s)
 {
-    if (n_inst <= 0)
+    // a workgroup per large instance, then 16 instances each; multiples of 8
+    // workgroups (one range per XCD)
+    const int n_small = n.n[0] + n.n[1] + n.n[2];
+    const int grid = (n.n[3] * p.n_ref + 7) / 8 * 8 + ((n_small * p.n_ref + 15) / 16 + 7) / 8 * 8;
+    if (grid <= 0)
         return XME_OK;
-    // a multiple of 8 workgroups (one range per XCD), 16 instances each
-    const int grid = ((n_inst + 15) / 16 + 7) / 8 * 8;
-    hipLaunchKernelGGL(mvc_kernel, dim3(grid), dim3(256), 0, s, p, d_desc, d_pus, d_inst, d_best, n_inst);
+    hipLaunchKernelGGL(mvc_kernel, dim3(grid), dim3(256), 0, s, p, d_desc, d_pus, d_inst, d_best, d_list, n_small, n.n[3]);
     XME_HIP(hipGetLastError());
     return XME_OK;
 }

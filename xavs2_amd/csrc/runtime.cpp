@@ -185,8 +185,8 @@ struct xme_plan {
     bool elim = false;
     int el_threads = 0;                // workgroup size of the elimination search
     bool el_few = false;               // fewer than 4 tasks per CU (xme_el_rows)
-    int32_t *d_sp_list = nullptr;      // sub-pel PU order: small PUs, then large ones
-    int n_sp_small = 0, n_sp_large = 0;
+    int32_t *d_sp_list = nullptr;      // PU order by sub-pel class
+    SubpelCounts n_sp = {};
     uint32_t *d_counters = nullptr;
     FrameDesc *d_desc = nullptr;
     int n_tasks = 0;
@@ -1073,14 +1073,14 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
     std::vector<int32_t> sp_list;      // lives until the arena uploads have been consumed
     {
         sp_list.reserve(pus.size());
-        for (int large = 0; large < 2; large++)
+        for (int cls = 0; cls < 4; cls++) {
             for (size_t i = 0; i < pus.size(); i++)
-                if (xme_subpel_large(pus[i].w, pus[i].h) == (large == 1))
+                if (xme_subpel_class(pus[i].w, pus[i].h) == cls)
                     sp_list.push_back((int32_t)i);
-        pl->n_sp_large = 0;
-        for (const DevPu &q : pus)
-            pl->n_sp_large += xme_subpel_large(q.w, q.h) ? 1 : 0;
-        pl->n_sp_small = (int)pus.size() - pl->n_sp_large;
+            pl->n_sp.n[cls] = (int)sp_list.size();
+        }
+        for (int cls = 3; cls > 0; cls--)
+            pl->n_sp.n[cls] -= pl->n_sp.n[cls - 1];
         up((void **)&pl->d_sp_list, sp_list.data(), sp_list.size() * sizeof(int32_t));
     }
     if (e == hipSuccess)
@@ -1370,14 +1370,13 @@ static int launch_search(xme_plan *pl, hipStream_t s)
 
 static int launch_all(xme_plan *pl, hipStream_t s)
 {
-    int rc = xme_launch_mvc(pl->p, pl->d_desc, pl->d_pus, pl->d_inst, pl->d_best, pl->n_inst, s);
+    int rc = xme_launch_mvc(pl->p, pl->d_desc, pl->d_pus, pl->d_inst, pl->d_best, pl->d_sp_list, pl->n_sp, s);
     if (rc)
         return rc;
     rc = launch_search(pl, s);
     if (rc)
         return rc;
-    return xme_launch_subpel(pl->p, pl->d_desc, pl->d_pus, pl->d_inst, pl->d_best, pl->d_sp_list, pl->n_sp_small,
-                             pl->n_sp_large, s);
+    return xme_launch_subpel(pl->p, pl->d_desc, pl->d_pus, pl->d_inst, pl->d_best, pl->d_sp_list, pl->n_sp, s);
 }
 
 extern "C" int xme_me_run(xme_plan *pl, const pel_t *cur, intptr_t i_cur, const xme_ref_desc *refs,
@@ -1447,7 +1446,7 @@ extern "C" int xme_me_time(xme_plan *pl, const pel_t *cur, intptr_t i_cur, const
         if (rc)
             break;
         XME_HIP(hipEventRecord(ev[4 * r + 0], s));
-        rc = xme_launch_mvc(pl->p, pl->d_desc, pl->d_pus, pl->d_inst, pl->d_best, pl->n_inst, s);
+        rc = xme_launch_mvc(pl->p, pl->d_desc, pl->d_pus, pl->d_inst, pl->d_best, pl->d_sp_list, pl->n_sp, s);
         if (rc)
             break;
         XME_HIP(hipEventRecord(ev[4 * r + 1], s));
@@ -1455,8 +1454,7 @@ extern "C" int xme_me_time(xme_plan *pl, const pel_t *cur, intptr_t i_cur, const
         if (rc)
             break;
         XME_HIP(hipEventRecord(ev[4 * r + 2], s));
-        rc = xme_launch_subpel(pl->p, pl->d_desc, pl->d_pus, pl->d_inst, pl->d_best, pl->d_sp_list, pl->n_sp_small,
-                               pl->n_sp_large, s);
+        rc = xme_launch_subpel(pl->p, pl->d_desc, pl->d_pus, pl->d_inst, pl->d_best, pl->d_sp_list, pl->n_sp, s);
         XME_HIP(hipEventRecord(ev[4 * r + 3], s));
     }
     if (rc == XME_OK)

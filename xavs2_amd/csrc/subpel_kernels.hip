@@ -14,10 +14,20 @@
 
 namespace {
 
-__constant__ int8_t c_spiral[9][2] = { { 0, 0 }, { 0, -1 }, { 0, 1 }, { -1, -1 }, { 1, -1 },
-                                       { -1, 0 }, { 1, 0 }, { -1, 1 }, { 1, 1 } };
-__constant__ int8_t c_spiral2[9][2] = { { 0, 0 }, { 0, -1 }, { -1, -1 }, { -1, 0 }, { -1, 1 },
-                                        { 0, 1 }, { 1, 1 }, { 1, 0 }, { 1, -1 } };
+constexpr int8_t kSpiral[9][2] = { { 0, 0 }, { 0, -1 }, { 0, 1 }, { -1, -1 }, { 1, -1 },
+                                   { -1, 0 }, { 1, 0 }, { -1, 1 }, { 1, 1 } };
+constexpr int8_t kSpiral2[9][2] = { { 0, 0 }, { 0, -1 }, { -1, -1 }, { -1, 0 }, { -1, 1 },
+                                    { 0, 1 }, { 1, 1 }, { 1, 0 }, { 1, -1 } };
+
+// A pattern's component a, 2 bits (offset + 1) per point: a lane's point comes
+// from a shift instead of a table read.
+constexpr uint32_t packed(const int8_t (&pat)[9][2], int a)
+{
+    uint32_t v = 0;
+    for (int k = 0; k < 9; k++)
+        v |= (uint32_t)(pat[k][a] + 1) << (2 * k);
+    return v;
+}
 
 // Picture and plane bytes in device memory.  The pointers come from the
 // frame descriptor as generic pointers; typing them global gives global (not
@@ -74,7 +84,10 @@ struct Stage {
     int bx, by, c0, step, stage;
     bool pmvr;
     int ctr_x, ctr_y;
-    const int8_t (*pat)[2];
+    uint32_t pat_x, pat_y;     // packed pattern
+
+    __device__ int px(int pos) const { return (int)((pat_x >> (2 * pos)) & 3u) - 1; }
+    __device__ int py(int pos) const { return (int)((pat_y >> (2 * pos)) & 3u) - 1; }
 };
 
 __device__ __forceinline__ void cand_mv(const Stage &st, int k, int &mx, int &my, bool &skip)
@@ -87,25 +100,25 @@ __device__ __forceinline__ void cand_mv(const Stage &st, int k, int &mx, int &my
             return;
         }
         const int pos = 1 + (k - st.c0) * st.step;
-        mx = st.bx + 2 * st.pat[pos][0];
-        my = st.by + 2 * st.pat[pos][1];
+        mx = st.bx + 2 * st.px(pos);
+        my = st.by + 2 * st.py(pos);
         return;
     }
     const int pos = 1 + k * st.step;
     if (st.pmvr) {
         if (iabs(st.bx - st.ctr_x) > 2 || iabs(st.by - st.ctr_y) > 2) {
-            mx = st.bx + st.pat[pos][0] * 2;
-            my = st.by + st.pat[pos][1] * 2;
+            mx = st.bx + st.px(pos) * 2;
+            my = st.by + st.py(pos) * 2;
             skip = iabs(mx - st.ctr_x) <= 2 && iabs(my - st.ctr_y) <= 2;
         } else {
-            mx = st.bx + st.pat[pos][0];
-            my = st.by + st.pat[pos][1];
+            mx = st.bx + st.px(pos);
+            my = st.by + st.py(pos);
             skip = iabs(mx - st.ctr_x) > 2 || iabs(my - st.ctr_y) > 2;
         }
         return;
     }
-    mx = st.bx + st.pat[pos][0];
-    my = st.by + st.pat[pos][1];
+    mx = st.bx + st.px(pos);
+    my = st.by + st.py(pos);
 }
 
 __device__ __forceinline__ int pack_cost_idx(int cost, int k)
@@ -214,9 +227,16 @@ __device__ int stage_min(const RefineCtx &c, const Stage &st, int n, int *start,
 
 constexpr int SP_WAVES = 4;
 
+// Workgroups of a class's instances: a multiple of 8 (one range per XCD).
+__host__ __device__ inline int subpel_blocks(int n_inst, int cls)
+{
+    const int per_wg = SP_WAVES * (cls == 0 ? 4 : cls == 1 ? 2 : 1);
+    return ((n_inst + per_wg - 1) / per_wg + 7) / 8 * 8;
+}
+
 // One workgroup of 4 waves takes either one instance of a PU of more than 64
-// tiles (the first n_large * n_ref workgroups, so the long instances start
-// first) or 4 instances of smaller PUs, one per wave.  Instances are walked
+// tiles (the first workgroups, so the long instances start first) or, one to
+// four per wave, instances of smaller PUs.  Instances are walked
 // reference-major (neighbouring PUs of one reference together) and each XCD
 // takes a contiguous range of workgroups, so the L2 of an XCD sees the plane
 // lines of neighbouring PUs back to back.
@@ -281,7 +301,8 @@ __device__ void refine(const DevParams &p, const FrameDesc *__restrict__ desc, c
         c.pmy = pu.mvp_y;
         Stage st;
         st.step = p.fast ? 2 : 1;
-        st.pat = p.fast ? c_spiral2 : c_spiral;
+        st.pat_x = p.fast ? packed(kSpiral2, 0) : packed(kSpiral, 0);
+        st.pat_y = p.fast ? packed(kSpiral2, 1) : packed(kSpiral, 1);
         st.pmvr = p.pmvr != 0;
         st.ctr_x = (pu.mvp_x >> 1) << 1;
         st.ctr_y = (pu.mvp_y >> 1) << 1;
@@ -331,52 +352,211 @@ __device__ void refine(const DevParams &p, const FrameDesc *__restrict__ desc, c
     }
 }
 
+// Sum over each aligned group of P = 4 or 8 lanes, in all of them.
+template <int P>
+__device__ __forceinline__ int tile_sum(int v)
+{
+    v = dpp_add<0xB1>(v);          // quad_perm [1,0,3,2]
+    v = dpp_add<0x4E>(v);          // quad_perm [2,3,0,1]
+    if (P == 8)
+        v = dpp_add<0x141>(v);     // row_half_mirror
+    return v;
+}
+
+// Minimum over the four groups of P lanes of each aligned 4 P lanes, in all of
+// them (equal within a group).
+template <int P>
+__device__ __forceinline__ int groups_min(int v)
+{
+    v = dpp_min<0x128>(v);         // row_ror:8
+    if (P == 4)
+        return dpp_min<0x124>(v);  // row_ror:4
+    return min(v, __shfl_xor(v, 16));
+}
+
+// PUs of at most P = 4 or 8 tiles: 4 P lanes per instance (a lane = a tile of
+// every fourth candidate), so a wave holds 4 or 2 instances and a stage of 9
+// candidates takes 3 steps and one of 8 takes 2, whose plane reads are in
+// flight together.  A wave per 8x8 instance took 2 steps for it alone, with 36
+// and 32 lanes at work.
+template <int P>
+__device__ __forceinline__ void refine_packed(const DevParams &p, const FrameDesc *__restrict__ desc,
+                                              const DevPu *__restrict__ pus, const DevInst *__restrict__ inst,
+                                              const uint64_t *__restrict__ best, int pu_i, int r, bool live)
+{
+    const int lane = threadIdx.x & 63, l = lane & (4 * P - 1), tile = l & (P - 1), g = l / P;
+    const int id = pu_i * p.n_ref + r;
+    const DevPu pu = pus[pu_i];
+    const uint4 vin = reinterpret_cast<const uint4 *>(inst)[id];
+    const DevInst in = __builtin_bit_cast(DevInst, vin);
+    const uint64_t key = best[id];
+    const bool ok = live && !in.status && key < XME_KEY_NONE;
+    const uint32_t order = (uint32_t)key;
+    int bmx, bmy;
+    if (order < XME_ORDER_RASTER) {
+        bmx = order == 0 ? in.mvc[0][0] : in.mvc[1][0];
+        bmy = order == 0 ? in.mvc[0][1] : in.mvc[1][1];
+    } else {
+        const int o = (int)order - XME_ORDER_RASTER, R2 = 2 * p.R;
+        bmx = in.omx + (o % R2) - p.R;
+        bmy = in.omy + (o / R2) - p.R;
+    }
+    int bx = 4 * bmx, by = 4 * bmy, bcost = (int)(key >> 32);
+    if (p.frac) {
+        const int tw = pu.w >> 2;
+        const bool has_tile = ok && tile < tw * (pu.h >> 2);
+        const int ty = has_tile ? (tile / tw) * 4 : 0, tx = has_tile ? (tile % tw) * 4 : 0;
+        RefineCtx c;
+        c.cur = (gbytes)desc->cur + (int64_t)pu.y * desc->i_cur + pu.x;
+        c.i_cur = desc->i_cur;
+        c.planes = desc->planes[r];
+        c.i_ref = desc->stride[r];
+        c.off = (int64_t)pu.y * c.i_ref + pu.x;
+        c.w = pu.w;
+        c.h = pu.h;
+        c.hadamard = p.hadamard != 0;
+        c.lambda = p.lambda;
+        c.pmx = pu.mvp_x;
+        c.pmy = pu.mvp_y;
+        uint32_t cr[4];
+#pragma unroll
+        for (int y = 0; y < 4; y++)
+            cr[y] = has_tile ? *(gdwords)(c.cur + (ty + y) * c.i_cur + tx) : 0u;
+        Stage st;
+        st.step = p.fast ? 2 : 1;
+        st.pat_x = p.fast ? packed(kSpiral2, 0) : packed(kSpiral, 0);
+        st.pat_y = p.fast ? packed(kSpiral2, 1) : packed(kSpiral, 1);
+        st.pmvr = p.pmvr != 0;
+        st.ctr_x = (pu.mvp_x >> 1) << 1;
+        st.ctr_y = (pu.mvp_y >> 1) << 1;
+        const int npts = p.fast ? 4 : 8;
+        for (int stage = 0; stage < (p.frac > 1 ? 2 : 1); stage++) {
+            st.stage = stage;
+            st.bx = bx;
+            st.by = by;
+            st.c0 = stage == 0 && c.hadamard ? 1 : 0;
+            const int n = st.c0 + npts;
+            int m = 0x7fffffff, start = 0x7fffffff;
+            auto step = [&](int k) {
+                int mx = 0, my = 0;
+                bool skip = true;
+                if (k < n)
+                    cand_mv(st, k, mx, my, skip);
+                int v = 0;
+                if (has_tile && !skip)
+                    v = tile_cost(cr, cand_ref(c, mx, my, ty, tx), c.i_ref, c.hadamard);
+                v = tile_sum<P>(v);
+                if (!skip) {
+                    const int cost = cand_cost(c, v, mx, my);
+                    if (k >= st.c0)
+                        m = min(m, pack_cost_idx(cost, k));
+                    else
+                        start = cost;
+                }
+            };
+            step(g);
+            if (n > 4)
+                step(4 + g);
+            if (n > 8)
+                step(8 + g);
+            m = groups_min<P>(m);
+            if (st.c0)
+                bcost = groups_min<P>(start);
+            if (m != 0x7fffffff && (m >> 4) < bcost) {
+                int mx, my;
+                bool skip;
+                cand_mv(st, m & 15, mx, my, skip);
+                bcost = m >> 4;
+                bx = mx;
+                by = my;
+            }
+        }
+    }
+    if (live && l == 0) {
+        xme_result res;
+        if (ok) {
+            res.cost = bcost;
+            res.bcost2 = (int)(key >> 32);
+            res.bmv_x = (int16_t)bx;
+            res.bmv_y = (int16_t)by;
+            res.bmv2_x = (int16_t)bmx;
+            res.bmv2_y = (int16_t)bmy;
+            res.mvcost = xme_weighted_cost(p.lambda, xme_mvbits(bx - pu.mvp_x) + xme_mvbits(by - pu.mvp_y));
+            res.status = (in.flags & 1) ? 2 : 0;
+        } else {
+            // _me_error (me.c:919-921, :1181): only the return value is defined
+            res.cost = XME_MAX_DISTORTION;
+            res.bcost2 = 0;
+            res.bmv_x = res.bmv_y = res.bmv2_x = res.bmv2_y = 0;
+            res.mvcost = 0;
+            res.status = 1;
+        }
+        desc->results[id] = res;
+    }
+}
+
 __global__ void __launch_bounds__(256) subpel_kernel(DevParams p, const FrameDesc *__restrict__ desc,
                                                      const DevPu *__restrict__ pus, const DevInst *__restrict__ inst,
                                                      const uint64_t *__restrict__ best,
-                                                     const int32_t *__restrict__ list, int n_small, int n_large)
+                                                     const int32_t *__restrict__ list, SubpelCounts n)
 {
     __shared__ int s_part[4 * 16];
     // Workgroup b runs on XCD b % 8.  The large instances take the first
     // blocks in dispatch order (spread over the XCDs), padded to a multiple of
-    // 8; the small ones then map to contiguous ranges per XCD.
-    const int n_large_wg = n_large * p.n_ref;
-    const int large_blocks = (n_large_wg + 7) / 8 * 8;
-    const int b = (int)blockIdx.x;
+    // 8; the classes of smaller ones then map to contiguous ranges per XCD.
+    int b = (int)blockIdx.x;
+    const int n_large_wg = n.n[3] * p.n_ref, large_blocks = (n_large_wg + 7) / 8 * 8;
+    const int32_t *large = list + n.n[0] + n.n[1] + n.n[2];
     if (b < large_blocks) {
         if (b < n_large_wg) {
-            const int r = b / n_large;
-            refine<true>(p, desc, pus, inst, best, list[n_small + b - r * n_large], r, s_part);
+            const int r = b / n.n[3];
+            refine<true>(p, desc, pus, inst, best, large[b - r * n.n[3]], r, s_part);
         }
         return;
     }
-    const int bs = b - large_blocks;                     // bs % 8 == b % 8
-    const int per_xcd = ((int)gridDim.x - large_blocks) / 8;
-    const int lb = (bs % 8) * per_xcd + bs / 8;
-    const int logical = __builtin_amdgcn_readfirstlane(lb * SP_WAVES + (int)(threadIdx.x >> 6));
-    if (logical >= n_small * p.n_ref)
+    b -= large_blocks;                                   // b % 8 is unchanged
+    int cls = 2;
+    for (; cls > 0 && b >= subpel_blocks(n.n[cls] * p.n_ref, cls); cls--)
+        b -= subpel_blocks(n.n[cls] * p.n_ref, cls);
+    const int n_cls = n.n[cls], per_wave = cls == 0 ? 4 : cls == 1 ? 2 : 1;
+    const int lb = (b % 8) * (subpel_blocks(n_cls * p.n_ref, cls) / 8) + b / 8;
+    const int first = __builtin_amdgcn_readfirstlane((lb * SP_WAVES + (int)(threadIdx.x >> 6)) * per_wave);
+    if (first >= n_cls * p.n_ref)
         return;
-    const int r = logical / n_small;
-    refine<false>(p, desc, pus, inst, best, list[logical - r * n_small], r, nullptr);
+    const int32_t *l = list + (cls == 2 ? n.n[0] + n.n[1] : cls == 1 ? n.n[0] : 0);
+    if (cls == 2) {
+        const int r = first / n_cls;
+        refine<false>(p, desc, pus, inst, best, l[first - r * n_cls], r, nullptr);
+        return;
+    }
+    const int at = first + (int)((threadIdx.x & 63) / (64 / per_wave));
+    const bool live = at < n_cls * p.n_ref;
+    const int i = live ? at : first, r = i / n_cls;
+    if (cls == 1)
+        refine_packed<8>(p, desc, pus, inst, best, l[i - r * n_cls], r, live);
+    else
+        refine_packed<4>(p, desc, pus, inst, best, l[i - r * n_cls], r, live);
 }
 
 } // namespace
 
-bool xme_subpel_large(int w, int h) { return (w >> 2) * (h >> 2) > 64; }
+int xme_subpel_class(int w, int h)
+{
+    const int tiles = (w >> 2) * (h >> 2);
+    return tiles <= 4 ? 0 : tiles <= 8 ? 1 : tiles <= 64 ? 2 : 3;
+}
 
 int xme_launch_subpel(const DevParams &p, const FrameDesc *d_desc, const DevPu *d_pus, const DevInst *d_inst,
-                      const uint64_t *d_best, const int32_t *d_list, int n_small, int n_large, hipStream_t s)
+                      const uint64_t *d_best, const int32_t *d_list, const SubpelCounts &n, hipStream_t s)
 {
-    // n_large * n_ref workgroups for the large PUs (rounded up to a multiple
-    // of 8), then SP_WAVES small instances per workgroup (a multiple of 8
-    // workgroups: one range per XCD)
-    const int large_blocks = (n_large * p.n_ref + 7) / 8 * 8;
-    const int small_blocks = ((n_small * p.n_ref + SP_WAVES - 1) / SP_WAVES + 7) / 8 * 8;
-    const int grid = large_blocks + small_blocks;
+    // a workgroup per large instance (rounded up to a multiple of 8), then the
+    // smaller classes, largest PUs first
+    int grid = (n.n[3] * p.n_ref + 7) / 8 * 8;
+    for (int cls = 0; cls < 3; cls++)
+        grid += subpel_blocks(n.n[cls] * p.n_ref, cls);
     if (grid <= 0)
         return XME_OK;
-    hipLaunchKernelGGL(subpel_kernel, dim3(grid), dim3(256), 0, s, p, d_desc, d_pus, d_inst, d_best, d_list, n_small,
-                       n_large);
+    hipLaunchKernelGGL(subpel_kernel, dim3(grid), dim3(256), 0, s, p, d_desc, d_pus, d_inst, d_best, d_list, n);
     XME_HIP(hipGetLastError());
     return XME_OK;
 }

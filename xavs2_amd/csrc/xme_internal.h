@@ -187,8 +187,18 @@ int xme_hip_fail(hipError_t e, const char *what);
     } while (0)
 
 // Launchers implemented in the .hip files.
+// Sub-pel refinement of every instance.  `d_list` holds the PU indices class
+// by class (xme_subpel_class: 0 at most 4 4x4 tiles, 1 at most 8, 2 at most 64,
+// 3 more), `n` how many of each.
+struct SubpelCounts {
+    int n[4];
+};
+int xme_subpel_class(int w, int h);
+int xme_launch_subpel(const DevParams &p, const FrameDesc *d_desc, const DevPu *d_pus, const DevInst *d_inst,
+                      const uint64_t *d_best, const int32_t *d_list, const SubpelCounts &n, hipStream_t s);
+// The MV candidate list of every instance; `d_list` and `n` as for the refinement.
 int xme_launch_mvc(const DevParams &p, const FrameDesc *d_desc, const DevPu *d_pus, DevInst *d_inst,
-                   uint64_t *d_best, int n_inst, hipStream_t s);
+                   uint64_t *d_best, const int32_t *d_list, const SubpelCounts &n, hipStream_t s);
 int xme_launch_fs(const DevParams &p, const FrameDesc *d_desc, const DevPu *d_pus, const DevInst *d_inst,
                   const FsTask *d_tasks, int n_tasks, const FsItem *d_items, const int32_t *d_item_insts,
                   uint64_t *d_best, uint32_t *d_counters, size_t lds_bytes, int grid, bool persistent, int kmax,
@@ -218,12 +228,6 @@ int xme_launch_elim(const DevParams &p, const FrameDesc *d_desc, const DevInst *
 // Raster costs of every candidate into the frame's cost map (diagnostics).
 int xme_launch_cost_map(const DevParams &p, const FrameDesc *d_desc, const DevPu *d_pus, const DevInst *d_inst,
                         int n_inst, hipStream_t s);
-// Sub-pel refinement of every instance.  `d_list` holds PU indices: the
-// first n_small PUs have at most 64 4x4 tiles (xme_subpel_large false), the
-// next n_large more; each part gets a kernel variant of its own.
-bool xme_subpel_large(int w, int h);
-int xme_launch_subpel(const DevParams &p, const FrameDesc *d_desc, const DevPu *d_pus, const DevInst *d_inst,
-                      const uint64_t *d_best, const int32_t *d_list, int n_small, int n_large, hipStream_t s);
 // Pattern searches (XME_ME_DIA, XME_ME_HEX) of every instance.  The six PU
 // size classes of xme_pattern_class (0: <= 16 pixel quads ... 5: > 256) run
 // as wave ranges, largest class first: range k holds class 5 - k with
