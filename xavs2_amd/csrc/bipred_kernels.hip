@@ -20,8 +20,19 @@
 
 namespace {
 
-__constant__ int8_t c_bi_spiral[9][2] = { { 0, 0 }, { 0, -1 }, { 0, 1 }, { -1, -1 }, { 1, -1 },
-                                         { -1, 0 }, { 1, 0 }, { -1, 1 }, { 1, 1 } };
+constexpr int8_t kSpiral[9][2] = { { 0, 0 }, { 0, -1 }, { 0, 1 }, { -1, -1 }, { 1, -1 },
+                                   { -1, 0 }, { 1, 0 }, { -1, 1 }, { 1, 1 } };
+
+// Spiral's component a at pos, from 2 bits (offset + 1) per point: a lane's
+// point costs a shift instead of a table read.
+__device__ __forceinline__ int spiral(int pos, int a)
+{
+    uint32_t v = 0;
+#pragma unroll
+    for (int k = 0; k < 9; k++)
+        v |= (uint32_t)(kSpiral[k][a] + 1) << (2 * k);
+    return (int)((v >> (2 * pos)) & 3u) - 1;
+}
 
 typedef const __attribute__((address_space(1))) uint8_t *gbytes;
 typedef const __attribute__((address_space(1))) uint32_t *gdwords;
@@ -68,15 +79,30 @@ __device__ __forceinline__ uint32_t avg4(uint32_t a, uint32_t b)
     return (a | b) - (((a ^ b) >> 1) & 0x7f7f7f7fu);
 }
 
-// Plane k of 16 without dynamic indexing of the kernel-argument array (a
-// select chain over uniform registers).
-__device__ __forceinline__ const uint8_t *pick_plane(const uint8_t *const (&pl)[16], int k)
+// The 16 + 16 plane pointers of a launch in LDS, where a lane picks the plane
+// of its candidate's phase with one read (a select chain over the kernel
+// arguments took 60 instructions a candidate; a dynamic index into them would
+// go to scratch).  Every thread of the workgroup calls load_planes.
+typedef uint64_t PlaneTab[32];
+
+__device__ __forceinline__ void load_planes(const SymPlanes &pl, PlaneTab &tab)
 {
-    const uint8_t *r = pl[0];
+    uint64_t v = 0;
+    if (threadIdx.x < 64) {
 #pragma unroll
-    for (int q = 1; q < 16; q++)
-        r = k == q ? pl[q] : r;
-    return r;
+        for (int k = 0; k < 16; k++) {
+            v = (int)threadIdx.x == k ? reinterpret_cast<uint64_t>(pl.p1[k]) : v;
+            v = (int)threadIdx.x == 16 + k ? reinterpret_cast<uint64_t>(pl.p2[k]) : v;
+        }
+        if (threadIdx.x < 32)
+            tab[threadIdx.x] = v;
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ const uint8_t *pick_plane(const PlaneTab &tab, int ref, int phase)
+{
+    return reinterpret_cast<const uint8_t *>(tab[16 * ref + phase]);
 }
 
 // scale_mv_skip (source/common/predict.h:148-151).
@@ -146,16 +172,24 @@ struct SymJob {
     gbytes cur;                // PU origin in the current picture
     int64_t i_cur, i_ref, off; // off: PU offset in the reference planes
     int w, h, tw, ntiles;
+    int ty0, tx0;              // the lane's first tile
     int mvp_x, mvp_y, dd, ds;
     bool neg, hadamard;
     int lambda;
     SymWindow win;
 };
 
+__device__ __forceinline__ void first_tile(SymJob &c, int P)
+{
+    const int t0 = (int)(threadIdx.x & 63) % P;
+    c.ty0 = (t0 / c.tw) * 4;
+    c.tx0 = (t0 % c.tw) * 4;
+}
+
 // ME_COST_QPEL_SYM (me.c:353-382) of candidate (mx, my), summed over the
 // lane's tiles t0, t0 + P, ...; returns -1 when the candidate has no cost
 // (an MV outside the window or a plane that is not built).
-__device__ __forceinline__ int sym_tiles(const SymJob &c, const SymPlanes &pl, int mx, int my, int t0, int P)
+__device__ __forceinline__ int sym_tiles(const SymJob &c, const PlaneTab &pl, int mx, int my, int t0, int P)
 {
     int sx = scale_mv(mx, c.dd, c.ds), sy = scale_mv(my, c.dd, c.ds);
     if (c.neg) {
@@ -164,15 +198,18 @@ __device__ __forceinline__ int sym_tiles(const SymJob &c, const SymPlanes &pl, i
     }
     if (!sym_legal(c.win, mx, my) || !sym_legal(c.win, sx, sy))
         return -1;
-    const uint8_t *a = pick_plane(pl.p1, ((my & 3) << 2) + (mx & 3));
-    const uint8_t *b = pick_plane(pl.p2, ((sy & 3) << 2) + (sx & 3));
+    const uint8_t *a = pick_plane(pl, 0, ((my & 3) << 2) + (mx & 3));
+    const uint8_t *b = pick_plane(pl, 1, ((sy & 3) << 2) + (sx & 3));
     if (a == nullptr || b == nullptr)
         return -1;
     const gbytes ga = (gbytes)a + c.off + (int64_t)(my >> 2) * c.i_ref + (mx >> 2);
     const gbytes gb = (gbytes)b + c.off + (int64_t)(sy >> 2) * c.i_ref + (sx >> 2);
-    int s = 0;
+    int s = 0, ty = c.ty0, tx = c.tx0;
     for (int t = t0; t < c.ntiles; t += P) {
-        const int ty = (t / c.tw) * 4, tx = (t % c.tw) * 4;
+        if (t != t0) {
+            ty = (t / c.tw) * 4;
+            tx = (t % c.tw) * 4;
+        }
         uint32_t cr[4], rr[4];
 #pragma unroll
         for (int y = 0; y < 4; y++) {
@@ -195,11 +232,11 @@ __device__ __forceinline__ void sym_cand(int stage, int pos0, int cx, int cy, bo
 {
     skip = false;
     if (stage == 0) {
-        mx = cx + 2 * c_bi_spiral[pos0 + k][0];
-        my = cy + 2 * c_bi_spiral[pos0 + k][1];
+        mx = cx + 2 * spiral(pos0 + k, 0);
+        my = cy + 2 * spiral(pos0 + k, 1);
         return;
     }
-    const int dx = c_bi_spiral[1 + k][0], dy = c_bi_spiral[1 + k][1];
+    const int dx = spiral(1 + k, 0), dy = spiral(1 + k, 1);
     if (pmvr) {
         const int ax = cx - ctr_x, ay = cy - ctr_y;
         if (ax > 2 || ax < -2 || ay > 2 || ay < -2) {
@@ -223,7 +260,7 @@ __device__ __forceinline__ void sym_cand(int stage, int pos0, int cx, int cy, bo
 // group's distortion sum.
 struct SymEval {
     const SymJob &c;
-    const SymPlanes &pl;
+    const PlaneTab &pl;
     __device__ __forceinline__ int tiles(int mx, int my, int t0, int P) const { return sym_tiles(c, pl, mx, my, t0, P); }
     __device__ __forceinline__ int cost(int s, int mx, int my) const
     {
@@ -269,7 +306,7 @@ struct SearchOut {
 };
 
 // xavs2_me_search_sym for job j, by the whole wave.
-__device__ SearchOut sym_search(const SymParams &p, const SymPlanes &pl, int64_t i_ref, const uint8_t *cur,
+__device__ SearchOut sym_search(const SymParams &p, const PlaneTab &pl, int64_t i_ref, const uint8_t *cur,
                                 int64_t i_cur, const xme_sym_job &j)
 {
     if (!sym_job_ok(p, j))
@@ -308,6 +345,7 @@ __device__ SearchOut sym_search(const SymParams &p, const SymPlanes &pl, int64_t
     int P = 1;
     while (P < c.ntiles && P < 64)
         P <<= 1;
+    first_tile(c, P);
     int bcost = XME_MAX_DISTORTION, bx = j.mv_x, by = j.mv_y;
     if (p.frac == 0) {
         // the start point alone; its cost is returned even when there is none
@@ -331,10 +369,12 @@ __global__ void __launch_bounds__(256) sym_kernel(SymParams p, SymPlanes pl, int
                                                   int64_t i_cur, const xme_sym_job *__restrict__ jobs, int n,
                                                   xme_sym_result *__restrict__ out)
 {
+    __shared__ PlaneTab tab;
+    load_planes(pl, tab);
     const int ji = job_index();
     if (ji >= n)
         return;
-    const SearchOut o = sym_search(p, pl, i_ref, cur, i_cur, jobs[ji]);
+    const SearchOut o = sym_search(p, tab, i_ref, cur, i_cur, jobs[ji]);
     if ((threadIdx.x & 63) == 0) {
         xme_sym_result res;
         res.cost = o.cost;
@@ -395,7 +435,7 @@ __device__ __forceinline__ uint32_t target4(uint32_t o, uint32_t p)
 // every PU size.
 struct BidEval {
     const SymJob &c;             // cur, strides, offset, tiles, window, lambda, switches
-    const uint8_t *const (&p1)[16];
+    const PlaneTab &pl;
     const uint32_t (&tgt)[4];
     gbytes gb;                   // the backward prediction at the PU origin
     bool bwd_legal;
@@ -404,17 +444,16 @@ struct BidEval {
     {
         if (!bwd_legal || !sym_legal(c.win, mx, my))
             return -1;
-        const uint8_t *a = pick_plane(p1, ((my & 3) << 2) + (mx & 3));
+        const uint8_t *a = pick_plane(pl, 0, ((my & 3) << 2) + (mx & 3));
         if (a == nullptr)           // the reference reads through a NULL plane here
             return -1;
         const gbytes ga = (gbytes)a + c.off + (int64_t)(my >> 2) * c.i_ref + (mx >> 2);
         int s = 0;
         if (t0 < c.ntiles) {
-            const int ty = (t0 / c.tw) * 4, tx = (t0 % c.tw) * 4;
             uint32_t rr[4];
 #pragma unroll
             for (int y = 0; y < 4; y++)
-                rr[y] = sym_load_dw(ga + (int64_t)(ty + y) * c.i_ref + tx);
+                rr[y] = sym_load_dw(ga + (int64_t)(c.ty0 + y) * c.i_ref + c.tx0);
             s = xme_tile_cost_rows(tgt, rr, c.hadamard);
         }
         for (int t = t0 + P; t < c.ntiles; t += P) {
@@ -439,7 +478,7 @@ struct BidEval {
 };
 
 // xavs2_me_search_bid for job j, by the whole wave.
-__device__ SearchOut bid_search(const SymParams &p, const SymPlanes &pl, int64_t i_ref, const uint8_t *cur,
+__device__ SearchOut bid_search(const SymParams &p, const PlaneTab &pl, int64_t i_ref, const uint8_t *cur,
                                 int64_t i_cur, const xme_bid_job &j)
 {
     const int lane = threadIdx.x & 63;
@@ -479,8 +518,9 @@ __device__ SearchOut bid_search(const SymParams &p, const SymPlanes &pl, int64_t
     while (P < c.ntiles && P < 64)
         P <<= 1;
     const int t0 = lane % P;
+    first_tile(c, P);
     const bool bwd_legal = sym_legal(c.win, j.bwd_x, j.bwd_y);
-    const uint8_t *p2 = pick_plane(pl.p2, ((j.bwd_y & 3) << 2) + (j.bwd_x & 3));
+    const uint8_t *p2 = pick_plane(pl, 1, ((j.bwd_y & 3) << 2) + (j.bwd_x & 3));
     if (bwd_legal && p2 == nullptr) {
         // the reference predicts from mc_luma here (me.c:1329-1335): not provided
         return SearchOut{ XME_MAX_DISTORTION, j.fwd_x, j.fwd_y, -1, 2 };
@@ -496,7 +536,7 @@ __device__ SearchOut bid_search(const SymParams &p, const SymPlanes &pl, int64_t
             tgt[y] = target4(*(gdwords)(c.cur + (ty + y) * i_cur + tx), sym_load_dw(gb + (int64_t)(ty + y) * i_ref + tx));
     }
     const int bid_bits = xme_weighted_cost(p.lambda, xme_mvbits(j.bwd_x - j.mvp2_x) + xme_mvbits(j.bwd_y - j.mvp2_y));
-    const BidEval ev{ c, pl.p1, tgt, gb, bwd_legal, j.mvp1_x, j.mvp1_y, bid_bits };
+    const BidEval ev{ c, pl, tgt, gb, bwd_legal, j.mvp1_x, j.mvp1_y, bid_bits };
     int bcost = XME_MAX_DISTORTION, bx = j.fwd_x, by = j.fwd_y;
     if (p.frac == 0) {
         bi_stage(ev, 0, 0, 1, j.fwd_x, j.fwd_y, false, 0, 0, P, bcost, bx, by);
@@ -518,10 +558,12 @@ __global__ void __launch_bounds__(256) bid_kernel(SymParams p, SymPlanes pl, int
                                                   int64_t i_cur, const xme_bid_job *__restrict__ jobs, int n,
                                                   xme_sym_result *__restrict__ out)
 {
+    __shared__ PlaneTab tab;
+    load_planes(pl, tab);
     const int ji = job_index();
     if (ji >= n)
         return;
-    const SearchOut o = bid_search(p, pl, i_ref, cur, i_cur, jobs[ji]);
+    const SearchOut o = bid_search(p, tab, i_ref, cur, i_cur, jobs[ji]);
     if ((threadIdx.x & 63) == 0) {
         xme_sym_result res;
         res.cost = o.cost;
@@ -607,6 +649,8 @@ __global__ void __launch_bounds__(256) bi_sym_kernel(SymParams p, GateParams g, 
                                                      const xme_bi_job *__restrict__ jobs, int n, int dist_fwd,
                                                      int dist_bwd, xme_bi_result *__restrict__ out)
 {
+    __shared__ PlaneTab tab;
+    load_planes(pl, tab);
     const int ji = job_index();
     if (ji >= n)
         return;
@@ -635,7 +679,7 @@ __global__ void __launch_bounds__(256) bi_sym_kernel(SymParams p, GateParams g, 
         sj.dist_fwd = (int16_t)dist_fwd;
         sj.dist_bwd = (int16_t)dist_bwd;
         sj.b_slice = 1;
-        const SearchOut o = sym_search(p, pl, i_ref, cur, i_cur, sj);
+        const SearchOut o = sym_search(p, tab, i_ref, cur, i_cur, sj);
         undef |= o.status != 0;
         cost = o.cost;
         mv_x = o.mv_x;
@@ -664,6 +708,8 @@ __global__ void __launch_bounds__(256) bi_bid_kernel(SymParams p, GateParams g, 
                                                      const xme_bi_job *__restrict__ jobs, int n, int dist_fwd,
                                                      int dist_bwd, xme_bi_result *__restrict__ out)
 {
+    __shared__ PlaneTab tab;
+    load_planes(pl, tab);
     const int ji = job_index();
     if (ji >= n)
         return;
@@ -692,7 +738,7 @@ __global__ void __launch_bounds__(256) bi_bid_kernel(SymParams p, GateParams g, 
         bj.mvp1_y = j.mvp1_y;
         bj.mvp2_x = j.mvp2_x;
         bj.mvp2_y = j.mvp2_y;
-        const SearchOut o = bid_search(p, pl, i_ref, cur, i_cur, bj);
+        const SearchOut o = bid_search(p, tab, i_ref, cur, i_cur, bj);
         undef |= o.status != 0;
         cost_bid = o.cost;
         fwd_x = o.mv_x;
@@ -728,6 +774,8 @@ __global__ void __launch_bounds__(256) dual_kernel(SymParams p, GateParams g, Sy
                                                    const xme_dual_job *__restrict__ jobs, int n, int r, int d_fwd,
                                                    int d_bwd, xme_dual_result *__restrict__ out)
 {
+    __shared__ PlaneTab tab;
+    load_planes(pl, tab);
     const int ji = job_index();
     if (ji >= n)
         return;
@@ -769,7 +817,7 @@ __global__ void __launch_bounds__(256) dual_kernel(SymParams p, GateParams g, Sy
         sj.dist_fwd = (int16_t)d_fwd;
         sj.dist_bwd = (int16_t)d_bwd;
         sj.b_slice = 0;
-        const SearchOut o = sym_search(p, pl, i_ref, cur, i_cur, sj);
+        const SearchOut o = sym_search(p, tab, i_ref, cur, i_cur, sj);
         undef |= o.status != 0;
         fx = o.mv_x;
         fy = o.mv_y;
