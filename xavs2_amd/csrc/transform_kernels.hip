@@ -43,7 +43,7 @@ struct QParams {
     int dscale, dshift;
 };
 
-enum { DO_FWD = 1, DO_QUANT = 2, DO_DEQUANT = 4, DO_INV = 8, DO_HALF = 16 };
+enum { DO_FWD = 1, DO_QUANT = 2, DO_DEQUANT = 4, DO_INV = 8, DO_HALF = 16, DO_WIDE = 32 };
 
 // The fused luma inter reconstruction (residual_kernel with FU = 1 or 2):
 // each tile's blocks are TUs of the record list {tu_x, tu_y, pu_x, pu_y, pu_w,
@@ -169,6 +169,44 @@ __host__ __device__ constexpr int rel_x(int x)
     return (x / N) * (N * N) + x % N;
 }
 
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+
+// The 16 values of a lane (rows rho(half, i) of its column) to memory as
+// int16, 8 bytes a store: the four lanes of a quad hold four rows of four
+// columns and exchange them, so that lane j of the quad stores row j of the
+// four columns.  The path is bound by memory, and 16 stores of 2 bytes a
+// lane kept it from its rate: 262144 blocks of 8x8 43.9 -> 33.4 us, of 16x16
+// 160.8 -> 131.0, of 32x32 388.7 -> 380.1 (4.2 TB/s of reads and writes; a copy
+// reaches 4.8).  The stores stream past the caches (8x8 40.9 us without); loads
+// that did so were slower (16x16 158.6).  Levels that are not 8-byte aligned, which the luma
+// reconstruction takes, keep the 2-byte stores (no DO_WIDE).
+// q_lane: the offset of (row rho(half, j), column 4 (col / 4)) for lane j.
+template <int N>
+__device__ __forceinline__ void store_quads(int16_t *dst, int64_t q_lane, int64_t b_lane, int nblk, int lane,
+                                            const int (&v)[16])
+{
+    constexpr int NB = 32 / N;
+    const bool o1 = lane & 1, o2 = lane & 2;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        // lane pairs: rows 0 and 2 of two columns to the even lane, 1 and 3 to the odd one
+        const uint32_t e = __builtin_amdgcn_perm((uint32_t)v[4 * g + 2], (uint32_t)v[4 * g], 0x05040100u);
+        const uint32_t o = __builtin_amdgcn_perm((uint32_t)v[4 * g + 3], (uint32_t)v[4 * g + 1], 0x05040100u);
+        const uint32_t keep = o1 ? o : e;
+        const uint32_t got = (uint32_t)__builtin_amdgcn_mov_dpp((int)(o1 ? e : o), 0xB1, 0xF, 0xF, false);
+        const uint32_t lo = o1 ? got : keep, hi = o1 ? keep : got;
+        const uint32_t r0 = __builtin_amdgcn_perm(hi, lo, 0x05040100u), r2 = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+        // pairs of pairs: rows 0, 1 of four columns to lanes 0, 1 and 2, 3 to lanes 2, 3
+        const uint32_t keep2 = o2 ? r2 : r0;
+        const uint32_t got2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)(o2 ? r0 : r2), 0x4E, 0xF, 0xF, false);
+        v2u w;
+        w[0] = o2 ? got2 : keep2;
+        w[1] = o2 ? keep2 : got2;
+        if (b_lane + (rho(0, 4 * g) / N) * NB < nblk)
+            __builtin_nontemporal_store(w, reinterpret_cast<v2u *>(dst + q_lane + rel_y<N>(rho(0, 4 * g))));
+    }
+}
+
 // Four prediction bytes at p (any alignment): the aligned dword pair around
 // them, realigned.  The dword after stays inside the plane's XME_PAD border.
 __device__ __forceinline__ uint32_t load4u(const uint8_t *p)
@@ -284,6 +322,7 @@ __global__ void __launch_bounds__(256) residual_kernel(const int16_t *__restrict
         // this lane's elements (rho(half, i), col): e_lane + rel_y(rho(0, i)),
         // in block b_lane + (rho(0, i) / N) * NB
         const int64_t e_lane = t * 1024 + rel_x<N>(col) + half * rel_y<N>(4);
+        const int64_t q_lane = t * 1024 + rel_x<N>(col & ~3) + half * rel_y<N>(4) + (col & 3) * N;
         const int64_t b_lane = t * BPT + col / N + (N == 4 ? half * NB : 0);
         // fused: this lane's 16 current and prediction bytes (tile row `col`,
         // columns 16 half .. 16 half + 15), kept for the reconstruction
@@ -520,10 +559,14 @@ __global__ void __launch_bounds__(256) residual_kernel(const int16_t *__restrict
                 }
             }
             // levels (or plain coefficients) out
+            if (FU == 3 || (mode & DO_WIDE)) {
+                store_quads<N>(level, q_lane, b_lane, nblk, lane, c);
+            } else {
 #pragma unroll
-            for (int i = 0; i < 16; i++)
-                if (b_lane + (rho(0, i) / N) * NB < nblk)
-                    level[e_lane + rel_y<N>(rho(0, i))] = (int16_t)c[i];
+                for (int i = 0; i < 16; i++)
+                    if (b_lane + (rho(0, i) / N) * NB < nblk)
+                        level[e_lane + rel_y<N>(rho(0, i))] = (int16_t)c[i];
+            }
             if ((mode & DO_QUANT) && nnz && lane < BPT && t * BPT + lane < nblk)
                 nnz[t * BPT + lane] = mine;
             if (mode & DO_INV) {
@@ -555,11 +598,12 @@ __global__ void __launch_bounds__(256) residual_kernel(const int16_t *__restrict
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int rv = xme_clip3(-RLIM, RLIM - 1, D[i] >> SI2);
-                if (!WL && recon && b_lane + (rho(0, i) / N) * NB < nblk)
-                    recon[e_lane + rel_y<N>(rho(0, i))] = (int16_t)rv;
+                v[i] = rv;
                 if constexpr (FU != 0)
                     s_res[wv][rho(half, i) * 32 + col] = (int16_t)rv;
             }
+            if (!WL && recon)
+                store_quads<N>(recon, q_lane, b_lane, nblk, lane, v);
         }
         if constexpr (WL) {
             // the inverse wavelet of the 32x32 residual in s_res: lanes 0..31
@@ -767,6 +811,8 @@ int launch_fu(int n, const int16_t *src, int16_t *level, int16_t *recon, int32_t
     std::call_once(g_tab_once, upload_tables);
     if (g_tab_err != hipSuccess)
         return xme_hip_fail(g_tab_err, "upload transform tables");
+    if ((reinterpret_cast<uintptr_t>(level) & 7) == 0)
+        mode |= DO_WIDE;
     // one wave per 32x32 tile of (32/n)^2 blocks (a 64x64 block's tile is its
     // wavelet low band); waves loop over tiles
     const int bpt = n >= 32 ? 1 : (32 / n) * (32 / n);
