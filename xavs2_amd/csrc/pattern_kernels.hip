@@ -1023,7 +1023,8 @@ __device__ __forceinline__ void pattern_wave(const DevParams &p, const FrameDesc
 }
 
 // Wave ranges of one launch, largest PUs first: range k holds PUs of
-// xme_pattern_class 5 - k, (64 / S) instance ids per wave from list[first[k]].
+// xme_pattern_class 5 - k, (64 / S) instance ids per wave from list[first[k]];
+// smaller PUs may lie in a range of more lanes than they need.
 struct PatLaunch {
     int end[6];      // first wave after range k
     int first[6];    // list index of range k's first id

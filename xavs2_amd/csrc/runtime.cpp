@@ -857,9 +857,31 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
         static const int per_wave[6] = { 1, 1, 2, 4, 8, 16 };
         int waves = 0;
         std::vector<int32_t> cls[6];
+        int n_cls[6] = {};
+        for (int i = 0; i < n_pu; i++)
+            n_cls[5 - xme_pattern_class(pus[i].w, pus[i].h)] += n_ref;
+        // A search is a chain of rounds of S points, so a small PU's instance
+        // is quicker with more lanes than its class has as long as the waves
+        // that makes still start together: smaller classes join class
+        // `least`, up to 3, while the launch has at most 2048 waves (2 per
+        // SIMD; 1024 and 4096 chose alike).  424x240, 8x8 PUs: UMH 343 -> 123
+        // us, TZ 308 -> 135, HEX 67 -> 48, DIA 83 -> 62; with more waves than
+        // that it loses (UMH, 1080p mixed PUs, class 2: 640 -> 753).  UMH's
+        // 16-point rounds fill 4 lanes four times over: 8 lanes are quicker
+        // at every size (1080p mixed 640 -> 606, 2160p 3711 -> 3644); TZ's
+        // are not (1080p mixed 485 -> 497).
+        auto waves_from = [&](int least) {
+            int n = 0, small = 0;
+            for (int k = 0; k < 6; k++)
+                (5 - k <= least ? small : n) += 5 - k <= least ? n_cls[k] : (n_cls[k] + per_wave[k] - 1) / per_wave[k];
+            return n + (small + per_wave[5 - least] - 1) / per_wave[5 - least];
+        };
+        int least = p.method == XME_ME_UMH ? 1 : 0;
+        while (least < 3 && waves_from(least + 1) <= 2048)
+            least++;
         for (int r = 0; r < n_ref; r++)
             for (int i = 0; i < n_pu; i++)
-                cls[5 - xme_pattern_class(pus[i].w, pus[i].h)].push_back(i * n_ref + r);
+                cls[5 - std::max(least, xme_pattern_class(pus[i].w, pus[i].h))].push_back(i * n_ref + r);
         for (int k = 0; k < 6; k++) {
             for (int32_t id : cls[k])
                 pat_list.push_back(id);
