@@ -10,8 +10,11 @@ bits (lambda factor 4 * 65536, MVP (0,0)), then half- and quarter-pel SATD
 refinement.  The whole frame is one persistent launch replayed from a HIP
 graph.
 
-Printed: one JSON line with candidate evaluations per second (batched path),
-the roofline of the integer-search kernel, the plain one-launch-per-PU-shape
+Printed: one JSON line with candidate evaluations per second (batched path:
+every legal candidate is decided; those whose bound from 4x4 sums already
+exceeds the best cost are not costed, with results equal to costing all),
+the roofline of the integer-search kernel (the share of SIMD cycles with a
+vector instruction, counted in the same run), the plain one-launch-per-PU-shape
 GPU path on the same job, per-frame latency p50/p99, and the CPU oracle timed
 on a bounded sample of the same job.  Side legs: the DIA, HEX and UMH
 pattern searches on the same frame, the residual transform, and the serving
@@ -29,7 +32,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 METRIC = "ME cand-evals/s + roofline frac, batched vs plain; p50/p99 frame-ME latency"
-VALU_PEAK_TABSDIFF = 256 * 4 * 16 * 2.4e9 * 4 / 1e12     # v_sad_u8 / v_qsad: 157.3 T absdiff/s
+VALU_PEAK_TCYCLES = 256 * 4 * 2.4e9 / 1e12      # 256 CUs of 4 SIMDs: T SIMD cycles/s with a vector instruction
 HBM_PEAK_GBS = 8000.0
 # The copy of known size that scales the HBM traffic counters, run beside the
 # search step in each counter pass.
@@ -921,7 +924,7 @@ def copy_probe(X, mib):
 
 
 def traffic_probe(X, args):
-    """Child of measure_traffic, run under rocprofv3 --pmc: the copy of
+    """Child of measure_counters, run under rocprofv3 --pmc: the copy of
     TRAFFIC_COPY_MIB MiB 3 times, then the bench's search step (the plan's
     graph) 3 times after one warm-up."""
     n = TRAFFIC_COPY_MIB << 20
@@ -938,12 +941,14 @@ def traffic_probe(X, args):
     print(json.dumps({"traffic_probe": "done"}), flush=True)
 
 
-def measure_traffic(args, timeout_s=240):
-    """roofline.traffic: HBM bytes per search step (its two persistent
-    dispatches), from two rocprofv3 --pmc children of this script in
-    --traffic-probe mode, FETCH_SIZE then WRITE_SIZE (KiB per dispatch), each
-    scaled by what the same counter reads for the copy of TRAFFIC_COPY_MIB MiB
-    in the same run.  Returns (bytes or None, details)."""
+def measure_counters(args, timeout_s=240):
+    """roofline.traffic and roofline.achieved: HBM bytes and busy VALU cycles
+    per search step (its persistent dispatches), from three rocprofv3 --pmc
+    children of this script in --traffic-probe mode.  FETCH_SIZE and
+    WRITE_SIZE (KiB per dispatch) are scaled by what the same counter reads
+    for the copy of TRAFFIC_COPY_MIB MiB in the same run; SQ_ACTIVE_INST_VALU
+    counts in units of 4 cycles.  Returns (bytes or None, cycles or None,
+    details)."""
     import csv
     import shutil
     import signal
@@ -951,13 +956,14 @@ def measure_traffic(args, timeout_s=240):
     import tempfile
     exe = shutil.which("rocprofv3")
     if exe is None:
-        return None, {"error": "rocprofv3 not found"}
+        return None, None, {"error": "rocprofv3 not found"}
     workload = ["--width", str(args.width), "--height", str(args.height), "--refs", str(args.refs), "--range",
                 str(args.range)] + (["--no-tune"] if args.no_tune else []) + (["--retune"] if args.retune else []) + \
                (["--pu-shape", args.pu_shape] if args.pu_shape else [])
     env = dict(os.environ, TMPDIR="/tmp")
     details, total = {}, 0.0
-    for counter in ("FETCH_SIZE", "WRITE_SIZE"):
+    cycles = None
+    for counter in ("FETCH_SIZE", "WRITE_SIZE", "SQ_ACTIVE_INST_VALU"):
         d = tempfile.mkdtemp(prefix="xme_traffic_", dir="/tmp")
         cmd = [exe, "--pmc", counter, "--output-format", "csv", "-d", d, "-o", "t", "--", sys.executable,
                os.path.abspath(__file__), "--serve-hw-queues", "0", "--traffic-probe"] + workload
@@ -970,31 +976,35 @@ def measure_traffic(args, timeout_s=240):
             os.killpg(proc.pid, signal.SIGKILL)
             proc.communicate()
             shutil.rmtree(d, ignore_errors=True)
-            return None, {"error": f"{counter} pass timed out"}
+            return None, None, {"error": f"{counter} pass timed out"}
         path = os.path.join(d, "t_counter_collection.csv")
         # the profiler may end with an error of its own after the program has
         # finished; its results are whole once the probe printed its last line
         if "traffic_probe" not in out or not os.path.exists(path):
             shutil.rmtree(d, ignore_errors=True)
-            return None, {"error": f"{counter} pass failed (exit {proc.returncode})"}
+            return None, None, {"error": f"{counter} pass failed (exit {proc.returncode})"}
         copy_kib, search_kib = [], {}
         with open(path) as f:
             for row in csv.DictReader(f):
                 name, v = row["Kernel_Name"], float(row["Counter_Value"])
                 if "copy_kernel" in name:
                     copy_kib.append(v)
-                elif "fs_kernel<true" in name:
-                    key = name[name.index("fs_kernel<"):]
+                elif "fs_kernel<true" in name or "elim_kernel<" in name:
+                    key = name[name.index("fs_kernel<" if "fs_kernel<" in name else "elim_kernel<"):]
                     search_kib.setdefault(key[:key.index(">") + 1], []).append(v)
         shutil.rmtree(d, ignore_errors=True)
         if not copy_kib or not search_kib:
-            return None, {"error": f"{counter} pass: no copy or search dispatch in the counters"}
+            return None, None, {"error": f"{counter} pass: no copy or search dispatch in the counters"}
+        if counter.startswith("SQ_"):
+            cycles = 4.0 * sum(float(np.median(v)) for v in search_kib.values())
+            details[counter] = {"per_dispatch": {k: float(np.median(v)) for k, v in search_kib.items()}}
+            continue
         scale = (TRAFFIC_COPY_MIB << 20) / (float(np.median(copy_kib)) * 1024.0)
         per_step = sum(float(np.median(v)) for v in search_kib.values()) * 1024.0 * scale
         details[counter] = {"kib_per_dispatch": {k: float(np.median(v)) for k, v in search_kib.items()},
                             "copy_kib": float(np.median(copy_kib)), "scale": scale, "bytes_per_step": per_step}
         total += per_step
-    return total, details
+    return total, cycles, details
 
 
 def setup_search(X, args):
@@ -1067,7 +1077,7 @@ def main():
     ap.add_argument("--copy-probe", type=int, default=0, metavar="MIB",
                     help="only run the 16-byte copy kernel over MIB MiB 20 times (HBM counter calibration)")
     ap.add_argument("--no-traffic", action="store_true",
-                    help="skip the two rocprofv3 --pmc passes that measure roofline.traffic")
+                    help="skip the three rocprofv3 --pmc passes that measure roofline.traffic and .achieved")
     ap.add_argument("--traffic-probe", action="store_true",
                     help="child mode of the traffic measurement: a copy and the search step, nothing printed "
                          "but a marker line")
@@ -1145,8 +1155,8 @@ def main():
 
     # roofline of the integer-search kernel: HIP events on its stream
     search_ms, job_ms, _ = plan.time(dcur, d_refs, stream.h, 5)
-    achieved = n_absdiff / (search_ms * 1e-3) / 1e12
-    log(f"search kernel {search_ms:.3f} ms, {achieved:.1f} T absdiff/s")
+    exhaustive_equiv = n_absdiff / (search_ms * 1e-3) / 1e12
+    log(f"search kernel {search_ms:.3f} ms, the work of {exhaustive_equiv:.1f} T absdiff/s by exhaustion")
 
     # plain path: one launch per PU shape, no persistent queue, no graph
     log("timing the plain path")
@@ -1185,10 +1195,11 @@ def main():
         threads = host["threads"]
         log(f"timing the CPU oracle on a sample ({threads} threads; host {host})")
         cpu = cpu_baseline((R, lam, 1, 2, 0, 0), refs, cur, pus, gpu_res, n_ref, args.cpu_seconds, threads, host)
-    traffic, traffic_detail = None, {"skipped": "--no-traffic"}
+    traffic, valu_cycles, traffic_detail = None, None, {"skipped": "--no-traffic"}
     if not args.no_traffic:
-        traffic, traffic_detail = measure_traffic(args)
-        log(f"traffic: {traffic} B per search step")
+        traffic, valu_cycles, traffic_detail = measure_counters(args)
+        log(f"counters: {traffic} B, {valu_cycles} VALU cycles per search step")
+    achieved = valu_cycles / (search_ms * 1e-3) / 1e12 if valu_cycles else None
 
     out = {
         "metric": METRIC,
@@ -1211,7 +1222,7 @@ def main():
                         "replayed from a HIP graph",
             "pu_refs": int(n_inst),
             "integer_candidates_per_step": int(n_cand),
-            "absdiffs_per_step": int(n_absdiff),
+            "exhaustive_absdiffs_per_step": int(n_absdiff),
             "lambda_factor": lam,
             "tiles_K_LC": {str(k): v for k, v in tiles.items()},
             "tiles_tuned_in_run": tuned_now,
@@ -1219,15 +1230,16 @@ def main():
         "roofline": {
             "bound": "valu",
             "achieved": achieved,
-            "peak": VALU_PEAK_TABSDIFF,
-            "unit": "Tabsdiff/s",
-            "frac": achieved / VALU_PEAK_TABSDIFF,
+            "peak": VALU_PEAK_TCYCLES,
+            "unit": "T SIMD cycles/s with a vector instruction (SQ_ACTIVE_INST_VALU, measured in this run)",
+            "frac": achieved / VALU_PEAK_TCYCLES if achieved else None,
+            "exhaustive_equivalent_tabsdiff_per_s": exhaustive_equiv,
             "traffic": traffic,
             "traffic_unit": "HBM bytes per search step, measured in this run: rocprofv3 --pmc FETCH_SIZE and "
                             "WRITE_SIZE on a child running the same step, each scaled by its reading for a "
                             f"{TRAFFIC_COPY_MIB} MiB copy in the same pass",
             "traffic_detail": traffic_detail,
-            "kernel": "integer full search: fs_kernel<true,8> (generic PUs) + fs_kernel<true,16> (PUs of <= 256 px), both persistent",
+            "kernel": "integer full search by elimination, elim_kernel (range > 64: fs_kernel), persistent",
             "kernel_ms": search_ms,
         },
         "plain": {"value": plain_value, "ms_per_step": plain_ms, "results_equal": plain_equal},

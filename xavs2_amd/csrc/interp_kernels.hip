@@ -368,10 +368,10 @@ __global__ void __launch_bounds__(NT) interp_kernel(Planes16 pl, InterpGeom g)
             for (int i = 0; i < 4; i++) {
                 int s = 2048 * 16;
 #pragma unroll
-                for (int m = 0; m < 4; m++)
-                    s = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2v, hp[m][i]),
-                                               short2v{ (short)(16 * c_taps[dy][2 * m]), (short)(16 * c_taps[dy][2 * m + 1]) }, s,
-                                               false);
+                for (int m = 0; m < 4; m++) {
+                    const short2v taps = { (short)(16 * c_taps[dy][2 * m]), (short)(16 * c_taps[dy][2 * m + 1]) };
+                    s = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2v, hp[m][i]), taps, s, false);
+                }
                 px[i] = (uint32_t)xme_clip3(0, 0xFFFFFF, s);
             }
             // the pixels are bytes 2

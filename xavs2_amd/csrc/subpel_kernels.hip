@@ -1,7 +1,9 @@
 // Sub-pel refinement (me_subpel_refine, source/encoder/me.c:479-579) and the
 // store of the full-pel result (me.c:1169-1173) for gfx950.
 //
-// One wave per (PU, ref).  The candidates of a refinement stage (the start
+// A wave per (PU, ref), a workgroup for PUs of more than 64 4x4 tiles, and 4 or
+// 2 PUs of at most 4 or 8 tiles per wave (2160p, 4 references: 434 -> 365 us,
+// bound by the latency of two dependent stages of plane reads).  The candidates of a refinement stage (the start
 // point and 8 half-pel points around the integer best, then 8 quarter-pel
 // points around the half-pel best) are independent, so a stage evaluates all
 // of them at once: lanes take (candidate, 4x4 tile) pairs, compute the tile's
