@@ -858,8 +858,11 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
         int waves = 0;
         std::vector<int32_t> cls[6];
         int n_cls[6] = {};
-        for (int i = 0; i < n_pu; i++)
-            n_cls[5 - xme_pattern_class(pus[i].w, pus[i].h)] += n_ref;
+        std::vector<int8_t> size_cls(n_pu);
+        for (int i = 0; i < n_pu; i++) {
+            size_cls[i] = (int8_t)xme_pattern_class(pus[i].w, pus[i].h);
+            n_cls[5 - size_cls[i]] += n_ref;
+        }
         // A search is a chain of rounds of S points, so a small PU's instance
         // is quicker with more lanes than its class has as long as the waves
         // that makes still start together: smaller classes join class
@@ -881,7 +884,7 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
             least++;
         for (int r = 0; r < n_ref; r++)
             for (int i = 0; i < n_pu; i++)
-                cls[5 - std::max(least, xme_pattern_class(pus[i].w, pus[i].h))].push_back(i * n_ref + r);
+                cls[5 - std::max<int>(least, size_cls[i])].push_back(i * n_ref + r);
         for (int k = 0; k < 6; k++) {
             for (int32_t id : cls[k])
                 pat_list.push_back(id);
@@ -1094,15 +1097,17 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
         e = plan_dev_alloc(pl, (void **)&pl->d_umh, sizeof(xme_umh_ctx) * pl->n_inst);
     std::vector<int32_t> sp_list;      // lives until the arena uploads have been consumed
     {
-        sp_list.reserve(pus.size());
-        for (int cls = 0; cls < 4; cls++) {
-            for (size_t i = 0; i < pus.size(); i++)
-                if (xme_subpel_class(pus[i].w, pus[i].h) == cls)
-                    sp_list.push_back((int32_t)i);
-            pl->n_sp.n[cls] = (int)sp_list.size();
+        std::vector<uint8_t> cls(pus.size());
+        for (size_t i = 0; i < pus.size(); i++) {
+            cls[i] = (uint8_t)xme_subpel_class(pus[i].w, pus[i].h);
+            pl->n_sp.n[cls[i]]++;
         }
-        for (int cls = 3; cls > 0; cls--)
-            pl->n_sp.n[cls] -= pl->n_sp.n[cls - 1];
+        int at[4] = {};
+        for (int k = 1; k < 4; k++)
+            at[k] = at[k - 1] + pl->n_sp.n[k - 1];
+        sp_list.resize(pus.size());
+        for (size_t i = 0; i < pus.size(); i++)
+            sp_list[at[cls[i]]++] = (int32_t)i;
         up((void **)&pl->d_sp_list, sp_list.data(), sp_list.size() * sizeof(int32_t));
     }
     if (e == hipSuccess)
