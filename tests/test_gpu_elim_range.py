@@ -1,0 +1,59 @@
+"""GPU parity of the batched full search (successive elimination) with the
+oracle and the plain plan where the best match lies just outside the search
+range: the rows after the last one of a window that is cut in row ranges."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests.test_gpu_me import LAM, compare, device_cur, oracle_ref, oracle_results
+from xavs2_amd import lib as X
+
+pytestmark = pytest.mark.gpu
+
+
+def check(ref, cur, pus, R, lam=LAM, plain=True, **kw):
+    """The batched plan's results, equal to the oracle's (and the plain plan's)."""
+    h, w = ref.shape
+    kw = dict(use_fractional_me=0, **kw)
+    dref = X.DeviceRef(w, h, frac=0)
+    dref.load(ref)
+    dcur = device_cur(cur)
+    plan = X.Plan(X.me_params(w, h, R, lam, **kw), X.make_pus(pus), 1)
+    plan.run(dcur, [dref])
+    got = plan.fetch()
+    compare(got, oracle_results(O.me_param(w, h, R, lam, **kw), pus, cur, [oracle_ref(ref, 0)], 1), pus, 1)
+    if plain:
+        other = X.Plan(X.me_params(w, h, R, lam, **kw), X.make_pus(pus), 1, X.PLAN_PLAIN)
+        other.run(dcur, [dref])
+        compare(got, other.fetch(), pus, 1)
+    return got
+
+
+@pytest.mark.parametrize("at", ["mvp", "origin"])
+@pytest.mark.parametrize("R", [18, 17, 19, 22, 23])
+def test_best_match_below_a_range_cut_in_rows(R, at):
+    """A PU whose two possible centres are 240 pixels apart is searched in row
+    ranges; at R = 18 the last one is the single row 35."""
+    w, h, x, y, mvp = 640, 512, 400, 300, (-240, -113)
+    rng = np.random.default_rng(R)
+    ref, cur = (rng.integers(0, 256, (h, w)).astype(np.uint8) for _ in range(2))
+    cx, cy = (x + mvp[0], y + mvp[1]) if at == "mvp" else (x, y)
+    block = cur[y:y + 16, x:x + 16] // 2
+    cur[y:y + 16, x:x + 16] = block
+    ref[cy:cy + 16, cx:cx + 16] = block + 2                     # the better candidate: the search centre
+    for dy in (R, R + 2):
+        r = ref.copy()
+        r[cy + dy:cy + dy + 16, cx + 5:cx + 21] = block         # an exact match outside the range
+        got = check(r, cur, [(x, y, 16, 16, 4 * mvp[0], 4 * mvp[1])], R)
+        assert (got["bmv_y"] < 4 * (cy - y + R)).all()
+
+
+@pytest.mark.parametrize("R", list(range(1, 65)))
+def test_every_range_with_cut_windows(R):
+    w, h = 640, 512
+    rng = np.random.default_rng(100 + R)
+    ref = rng.integers(0, 256, (h, w)).astype(np.uint8)
+    cur = np.roll(ref, (5, 3), (0, 1)) ^ rng.integers(0, 8, (h, w)).astype(np.uint8)
+    pus = [(400, 300, 16, 16, -960, -452), (320, 64, 8, 8, -600, 700), (192, 192, 12, 16, 33, -900),
+           (448, 400, 32, 32, -700, -400), (256, 256, 64, 64, 40, -24)]
+    check(ref, cur, pus, R, plain=False)

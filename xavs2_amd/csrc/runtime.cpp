@@ -460,7 +460,9 @@ static bool el_cuts(const DevParams &p, const std::vector<DevPu> &pus, const std
 {
     const int K = xme_el_rows(p.R, false, 4, 4), R2 = 2 * p.R;      // the most any PU takes
     for (int splits = 1; splits <= 2 || members.size() == 1; splits *= 2) {
-        const int per = std::max(K, (R2 + splits - 1) / splits);
+        // an even count: the kernel takes candidate rows in pairs, and does not
+        // look at each row of a pair when R is even
+        const int per = std::max(K, ((R2 + splits - 1) / splits + 1) & ~1);
         const size_t before = out.size();
         size_t need = 0;
         for (int lo = 0; lo < R2 && need <= cap; lo += per) {
