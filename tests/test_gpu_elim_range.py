@@ -1,6 +1,7 @@
 """GPU parity of the batched full search (successive elimination) with the
 oracle and the plain plan where the best match lies just outside the search
-range: the rows after the last one of a window that is cut in row ranges."""
+range: the rows after the last one of a window that is cut in row ranges, and
+columns right of it where costs are near the largest."""
 import numpy as np
 import pytest
 
@@ -57,3 +58,24 @@ def test_every_range_with_cut_windows(R):
     pus = [(400, 300, 16, 16, -960, -452), (320, 64, 8, 8, -600, 700), (192, 192, 12, 16, 33, -900),
            (448, 400, 32, 32, -700, -400), (256, 256, 64, 64, 40, -24)]
     check(ref, cur, pus, R, plain=False)
+
+
+@pytest.mark.parametrize("R", [24, 40, 48])
+def test_largest_costs(R):
+    """64x64 PUs, white against black, at the largest lambda and far from their
+    MVP: every candidate costs 1044476 + 12799, the origin's as much and the
+    clipped MVP's 4 more.  Nothing is eliminated, and the columns right of the
+    range hold cheaper pixels."""
+    w, h, x, y = 256, 256, 64, 64
+    cur = np.full((h, w), 255, np.uint8)
+    ref = np.zeros((h, w), np.uint8)
+    # one pixel of 4 in every block at a displacement of the range, none in
+    # the block one column and row before it
+    for px in (x + 63 - R, x + 127 - R):
+        for py in (y + 63 - R, y + 127 - R):
+            ref[py, px] = 4
+    ref[:, x + 63 + R:] = 100                                   # seen from displacement R on
+    m = -4 * (R + 7)                                            # the window starts at -(R + 1)
+    pus = [(x, y, 64, 64, -3000 - 2 * i, -3000 + 2 * i) for i in range(48)]
+    got = check(ref, cur, pus, R, lam=(1 << 24) - 1, plain=False, mv_range_x=(m, 4 * (R + 60)), mv_range_y=(m, 4 * (R + 60)))
+    assert (got["bmv_x"] == 0).all() and (got["bmv_y"] == 0).all()

@@ -56,7 +56,13 @@ struct WaveArea {
 };
 static_assert(sizeof(WaveArea) == XME_EL_WAVE_BYTES, "plan and kernel agree on the LDS of a wave");
 
-constexpr uint32_t kNever = 1u << 20;      // bound term of a candidate that cannot be chosen
+// Bound term of a candidate that cannot be chosen: above every cost (the SAD
+// of 64 x 64 pixels and the rate of two 29-bit vector differences at the
+// largest lambda).  A column's and a row's, with the largest bound between
+// them, fit the 27 bits that a tile's key gives them.
+constexpr uint32_t kNever = 1u << 21;
+static_assert(64 * 64 * 255 + (((uint64_t)(1 << 24) * 2 * 29) >> 16) < kNever, "a threshold never reaches the term");
+static_assert(2ull * kNever + 64 * 64 * 255 < 1u << 27, "and the term fits the key");
 
 template <int CTRL>
 __device__ __forceinline__ uint32_t row_min_step(uint32_t v)
