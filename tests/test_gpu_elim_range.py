@@ -1,7 +1,7 @@
 """GPU parity of the batched full search (successive elimination) with the
 oracle and the plain plan where the best match lies just outside the search
-range: the rows after the last one of a window that is cut in row ranges, and
-columns right of it where costs are near the largest."""
+range: candidate columns that a row of lanes has beyond 2R, the rows after the
+last one of a window that is cut in row ranges, and costs near the largest."""
 import numpy as np
 import pytest
 
@@ -28,6 +28,24 @@ def check(ref, cur, pus, R, lam=LAM, plain=True, **kw):
         other.run(dcur, [dref])
         compare(got, other.fetch(), pus, 1)
     return got
+
+
+@pytest.mark.parametrize("pw,ph", [(8, 8), (16, 4), (4, 16), (8, 4), (4, 8), (4, 4), (16, 16), (32, 32)])
+@pytest.mark.parametrize("R", [33, 34, 40, 46, 48, 57])
+def test_best_match_right_of_the_range(R, pw, ph):
+    """The columns of a row of lanes end at 64 or 128, those of the range at 2R.
+    Every row of these pictures is the same, and each PU matches exactly at the
+    first column after the range, or at one that a row of 16 lanes wholly
+    outside it starts with."""
+    w, h = 384, 192
+    for dx in sorted({R, R + 2, 96 - R, 97 - R}):
+        if dx < R:
+            continue
+        row = np.random.default_rng(dx).integers(0, 256, w + 128).astype(np.uint8)
+        ref, cur = np.tile(row[:w], (h, 1)), np.tile(row[dx:dx + w], (h, 1))
+        pus = [(x, y, pw, ph, 0, 0) for y in (64, 96) for x in range(64, 224, 32)]
+        got = check(ref, cur, pus, R, plain=False)
+        assert (got["bmv_x"] < 4 * R).all()
 
 
 @pytest.mark.parametrize("at", ["mvp", "origin"])

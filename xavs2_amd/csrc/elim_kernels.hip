@@ -385,7 +385,8 @@ struct Item {
 
     // The smallest cost among the tiles of the smallest bounds, one per row of
     // 16 lanes (PUs of at most 16 dwords) or one for the wave: the lanes share
-    // the tile's pixels.
+    // the tile's pixels.  A row of lanes that owns only columns from 2 R on
+    // has no tile to offer.
     __device__ __forceinline__ uint32_t probe(uint32_t kmin, int row, int quad) const
     {
         constexpr bool QUARTER = ONE && NX * 4 * NY <= 16;
@@ -425,7 +426,7 @@ struct Item {
             for (int k = 0; k < 8; k++)
                 sad[k] = (uint32_t)group_sum((int)sad[k], 64);
         }
-        const uint32_t key = tile_key(trow, tcol, sad);
+        const uint32_t key = (best >> 5) < kNever ? tile_key(trow, tcol, sad) : 0xFFFFFFFFu;
         return QUARTER ? wave_min(key >> 3) : (uint32_t)__builtin_amdgcn_readlane((int)(key >> 3), 63);
     }
 
