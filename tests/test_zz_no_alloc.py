@@ -67,3 +67,22 @@ def test_static_search_refuses_a_plan_beyond_the_scratch():
     rc, _ = static_search(X.me_params(w, h, 16, LAM), pus, 8, dcur, [ref] * 8)
     assert rc == X.XME_ERR_BUDGET
     assert b"static scratch" in X.lib().xme_last_error()
+
+
+def test_static_search_of_a_job_near_the_scratch_size():
+    """8x8 PUs over 8192x4096 against 3 references: 1.57 M instances, whose
+    exhaustive plan fits the scratch (about 55 of 64 MiB) and whose elimination
+    plan does not (70 MiB)."""
+    w, h = 8192, 4096
+    img = np.tile(synth.smooth_field(512, 256, seed=7), (h // 256, w // 512))
+    ref = X.DeviceRef(w, h, frac=0)
+    ref.load(img)
+    dcur = device_cur(np.roll(img, (1, 1), (0, 1)))
+    pus = np.zeros((h // 8) * (w // 8), dtype=X.PU_DTYPE)
+    pus["x"] = np.tile(np.arange(0, w, 8), h // 8)
+    pus["y"] = np.repeat(np.arange(0, h, 8), w // 8)
+    pus["w"] = pus["h"] = 8
+    prm = X.me_params(w, h, 2, LAM, use_fractional_me=0)
+    rc, got = static_search(prm, pus, 3, dcur, [ref] * 3)
+    assert rc == 0, X.lib().xme_last_error()
+    assert np.array_equal(got, plan_search(prm, pus, 3, dcur, [ref] * 3))

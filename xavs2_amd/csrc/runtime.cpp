@@ -639,7 +639,8 @@ static hipError_t plan_zero(xme_plan *pl, void *d, size_t n)
 }
 
 static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int n_pu, int n_ref, int mode,
-                            uint8_t *arena, size_t arena_cap, hipStream_t arena_stream, xme_plan **out);
+                            uint8_t *arena, size_t arena_cap, hipStream_t arena_stream, xme_plan **out,
+                            bool may_elim = true);
 
 extern "C" int xme_plan_create(const xme_me_params *prm, const xme_pu *pus_in, int n_pu, int n_ref, int mode,
                                xme_plan **out)
@@ -648,7 +649,7 @@ extern "C" int xme_plan_create(const xme_me_params *prm, const xme_pu *pus_in, i
 }
 
 static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int n_pu, int n_ref, int mode,
-                            uint8_t *arena, size_t arena_cap, hipStream_t arena_stream, xme_plan **out)
+                            uint8_t *arena, size_t arena_cap, hipStream_t arena_stream, xme_plan **out, bool may_elim)
 {
     if (!prm || !pus_in || !out || n_pu <= 0 || n_ref <= 0 || n_ref > XME_MAX_REFS ||
         (mode != XME_PLAN_BATCHED && mode != XME_PLAN_PLAIN)) {
@@ -807,7 +808,7 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
     // LDS with their sums; the others, plain plans and the tuner (which times
     // the exhaustive tiles) search exhaustively.
     std::vector<ElCut> cuts;
-    if (p.method == XME_ME_FS && mode == XME_PLAN_BATCHED && p.R <= XME_EL_MAX_R && !xme_tune_forced()) {
+    if (may_elim && p.method == XME_ME_FS && mode == XME_PLAN_BATCHED && p.R <= XME_EL_MAX_R && !xme_tune_forced()) {
         // one task per 64x64 CTU and reference (all PU shapes together); per
         // quarter CTU when that gives fewer tasks than CUs (1080p 16x16 PUs,
         // R = 32, 510 CTUs: 53 us whole, 85 us in quarters; 720p, R = 8, 240
@@ -1143,6 +1144,12 @@ static int plan_create_impl(const xme_me_params *prm, const xme_pu *pus_in, int 
         int rc;
         if (pl->arena)
             (void)hipStreamSynchronize(arena_stream);   // copies already queued read the host lists
+        if (pl->arena && pl->arena_used > pl->arena_cap && pl->elim) {
+            // the exhaustive search's items hold several instances each: its
+            // plan takes about 10 bytes less per instance
+            plan_free(pl);
+            return plan_create_impl(prm, pus_in, n_pu, n_ref, mode, arena, arena_cap, arena_stream, out, false);
+        }
         if (pl->arena && pl->arena_used > pl->arena_cap) {
             xme_set_error("xme_me_search_static: the job's plan needs more than the %zu bytes of static scratch "
                           "(fewer PUs or references per call)", pl->arena_cap);
