@@ -24,6 +24,9 @@
 //    When fewer than 33 tiles are left, 2 to 64 lanes share a tile's rows.
 //  * Before a band's tiles are listed, the tile with the smallest bound is
 //    costed by the whole wave; its cost is the next bound's threshold.
+//  * Where the bounds let most of a band pass (noise), the rest of the item is
+//    costed in strips, every candidate of it: 4 columns x 8 rows a lane, each
+//    window row read once.
 //
 // Bound: VALU issue (83 % busy at 2160p): an 8x8 PU's band of 2048 candidates
 // takes about 150 instructions of bounds, 75 of listing and 0.8 x 240 of exact
@@ -34,12 +37,17 @@
 // -> 825, 16x16 1150 -> 590, 32x32 1100 -> 625, 64x64 1045 -> 735, mixed PUs
 // 1345 -> 695 us (4 references 4.90 -> 2.9 ms); with random MVPs (+-10 px)
 // 1510 -> 870; 1080p 16x16, R = 32: 92 -> 51; 424x240 mixed, R = 16: 170 -> 52
-// us.  On pure noise, where nothing is eliminated, it is the slower one (1080p,
-// R = 64: 8x8 427 -> 577, 16x16 331 -> 415, mixed 566 -> 474 us).
+// us.  On pure noise, where nothing is eliminated, exhaustive -> tiles alone ->
+// this (1080p, R = 64): 8x8 417 -> 577 -> 425 us, 16x16 330 -> 410 -> 345, 32x32
+// 325 -> 381 -> 348, 64x64 303 -> 406 -> 370 (a wave's one or two items there
+// begin with bounds), mixed 560 -> 466 -> 374; R = 32, 8x8 117 -> 177 -> 136;
+// 2160p mixed 1330 -> 1660 -> 1341, and with noise of 16 levels over structure
+// 1330 -> 1574 -> 1405.
 #include "xme_dpp.h"
 #include "xme_internal.h"
 
 #include <mutex>
+#include <type_traits>
 
 namespace {
 
@@ -322,12 +330,29 @@ struct TaskView {
     int wx0, wy0, cx0, cy0;
 };
 
-// What a wave keeps between items: what its rate terms were made for, and the
-// bands it searches without bounds after one that eliminated nearly nothing.
+// Where more than kDenseNum / kDenseDen of a band's tiles pass the bounds, the
+// bands after it are searched without them.  With STRIPS (el_strips) every
+// candidate of the rest of the item is costed by dense_rows, and so are those
+// of the wave's next 3 items, then 15; else the tiles of the next 3 bands are
+// all listed.  4 / 5 is quicker on noise of 16 levels over structure (2160p
+// mixed PUs, 1 reference 1377 us against 1388) but costs pictures with less (4
+// references, noise of 3: 3180 us without strips, 3199 at 9 / 10, 3245 at 4 / 5).
+constexpr int kDenseNum = 9, kDenseDen = 10, kDenseRun = 15;
+
+// What a wave keeps between items: what its rate terms were made for, the items
+// (or bands) it still searches without bounds after one that eliminated nearly
+// nothing, and how many such the last one led to.
 struct WaveState {
     bool ok;
     int cx, cy, px, py;
-    int dense;
+    int dense, run;
+};
+
+// An instance's search box: the legal candidate columns, and whether every
+// candidate is legal.
+struct Box {
+    int lox, hix;
+    bool all_legal;
 };
 
 // One item: the candidate rows [row0, row0 + nrows) of one instance.  ONE: its
@@ -493,14 +518,58 @@ struct Item {
     }
 };
 
-template <int K, int NX, int NY, bool ONE>
-__device__ __forceinline__ void el_item(const DevParams &p, const TaskView &v, const DevPu &pu, const DevInst &in,
-                                        int inst_id, int row0, int nrows, int lc_log2, uint64_t key0,
-                                        uint64_t *__restrict__ best, WaveArea *__restrict__ wa, WaveState &rs)
+// The box of an instance, and its rate terms in the wave's LDS.
+__device__ __forceinline__ Box rate_terms(const DevParams &p, const DevPu &pu, const DevInst &in,
+                                          WaveArea *__restrict__ wa, WaveState &rs)
+{
+    const int lane = threadIdx.x & 63, R = p.R, R2 = 2 * p.R;
+    // The packed range check equals the box test while |MV| < 8192; the bound
+    // drops illegal candidates only then (the exact costs check each one).
+    const MvWindow mw = xme_mv_window(p, pu.x, pu.y, pu.w, pu.h);
+    const bool boxed = mw.min_fpel[0] > -8192 && mw.max_fpel[0] < 8192 && mw.min_fpel[1] > -8192 &&
+                       mw.max_fpel[1] < 8192 && in.omx - R > -8192 && in.omx + R < 8192 && in.omy - R > -8192 &&
+                       in.omy + R < 8192;
+    Box box;
+    box.all_legal = boxed && in.omx - R >= mw.min_fpel[0] && in.omx + R - 1 <= mw.max_fpel[0] &&
+                    in.omy - R >= mw.min_fpel[1] && in.omy + R - 1 <= mw.max_fpel[1];
+    box.lox = boxed ? mw.min_fpel[0] - in.omx + R : 0;
+    box.hix = boxed ? min(R2 - 1, mw.max_fpel[0] - in.omx + R) : R2 - 1;
+    if (rs.ok && box.all_legal && rs.cx == in.omx && rs.cy == in.omy && rs.px == pu.mvp_x && rs.py == pu.mvp_y)
+        return box;
+    // ME_COST_IPEL's rate (me.c:187-192) is (lambda * (bits x + bits y)) >> 16;
+    // lambda < 2^24 and the bit counts are small, so the sum of the two
+    // products is the same (below 2^31)
+    const int loy = boxed ? mw.min_fpel[1] - in.omy + R : 0;
+    const int hiy = boxed ? min(R2 - 1, mw.max_fpel[1] - in.omy + R) : R2 - 1;
+    for (int i = lane; i < min(R2 + 16, kMaxR2); i += 64) {
+        const uint32_t ty = __umul24((uint32_t)p.lambda, (uint32_t)xme_mvbits(4 * (in.omy + i - R) - pu.mvp_y));
+        const uint32_t tn = __umul24((uint32_t)p.lambda, (uint32_t)xme_mvbits(4 * (in.omy + i + 1 - R) - pu.mvp_y));
+        const bool never = i > hiy || i + 1 < loy;      // both rows of the pair
+        wa->xt[i] = __umul24((uint32_t)p.lambda, (uint32_t)xme_mvbits(4 * (in.omx + i - R) - pu.mvp_x));
+        wa->yt[i] = ty;
+        wa->yp[i] = ((never ? kNever : min(ty, tn) >> 16) << 5) | (uint32_t)(i & 31);
+    }
+    rs.ok = box.all_legal;
+    rs.cx = in.omx;
+    rs.cy = in.omy;
+    rs.px = pu.mvp_x;
+    rs.py = pu.mvp_y;
+    wave_sync();
+    return box;
+}
+
+// The bands of an item by elimination, from the middle one outwards, up to the
+// first whose bounds eliminate nearly nothing: true when there is one.  Left to
+// search are then the candidate rows below end_lo and those from begin_hi on.
+template <int K, int NX, int NY, bool ONE, bool STRIPS>
+__device__ __forceinline__ bool el_item(const DevParams &p, const TaskView &v, const DevPu &pu, const DevInst &in,
+                                       const Box &box, int row0, int nrows, int lc_log2, uint32_t T,
+                                       WaveArea *__restrict__ wa, WaveState &rs, uint32_t &bc, uint32_t &bo,
+                                       int &end_lo, int &begin_hi)
 {
     int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));      // keeps what follows from the lane inside this item's code
-    Item<K, NX, NY, ONE> I{ p, v, pu, in, wa, lane, 0, 0, false, nullptr };
+    Item<K, NX, NY, ONE> I{ p, v, pu, in, wa, lane, 0, 0, box.all_legal, nullptr };
     const int R = p.R, R2 = 2 * p.R;
     const int bx = I.bx = pu.x + in.omx - R - v.wx0, by = I.by = pu.y + in.omy - R - v.wy0;
     constexpr int CP = (NX + 1) / 2;           // dwords of a sub-block row of a chunk
@@ -521,40 +590,6 @@ __device__ __forceinline__ void el_item(const DevParams &p, const TaskView &v, c
         }
         wa->cs[s] = s0 | (s1 << 16);
     }
-
-    // The packed range check equals the box test while |MV| < 8192; the bound
-    // drops illegal candidates only then (the exact costs check each one).
-    int lox, hix;
-    {
-        const MvWindow mw = xme_mv_window(p, pu.x, pu.y, pu.w, pu.h);
-        const bool boxed = mw.min_fpel[0] > -8192 && mw.max_fpel[0] < 8192 && mw.min_fpel[1] > -8192 &&
-                           mw.max_fpel[1] < 8192 && in.omx - R > -8192 && in.omx + R < 8192 && in.omy - R > -8192 &&
-                           in.omy + R < 8192;
-        const bool all_legal = I.all_legal = boxed && in.omx - R >= mw.min_fpel[0] && in.omx + R - 1 <= mw.max_fpel[0] &&
-                                             in.omy - R >= mw.min_fpel[1] && in.omy + R - 1 <= mw.max_fpel[1];
-        lox = boxed ? mw.min_fpel[0] - in.omx + R : 0;          // legal candidate columns
-        hix = boxed ? min(R2 - 1, mw.max_fpel[0] - in.omx + R) : R2 - 1;
-        if (!(rs.ok && all_legal && rs.cx == in.omx && rs.cy == in.omy && rs.px == pu.mvp_x && rs.py == pu.mvp_y)) {
-            // ME_COST_IPEL's rate (me.c:187-192) is (lambda * (bits x + bits y)) >> 16;
-            // lambda < 2^24 and the bit counts are small, so the sum of the two
-            // products is the same (below 2^31)
-            const int loy = boxed ? mw.min_fpel[1] - in.omy + R : 0;
-            const int hiy = boxed ? min(R2 - 1, mw.max_fpel[1] - in.omy + R) : R2 - 1;
-            for (int i = lane; i < min(R2 + K, kMaxR2); i += 64) {
-                const uint32_t ty = __umul24((uint32_t)p.lambda, (uint32_t)xme_mvbits(4 * (in.omy + i - R) - pu.mvp_y));
-                const uint32_t tn = __umul24((uint32_t)p.lambda, (uint32_t)xme_mvbits(4 * (in.omy + i + 1 - R) - pu.mvp_y));
-                const bool never = i > hiy || i + 1 < loy;      // both rows of the pair
-                wa->xt[i] = __umul24((uint32_t)p.lambda, (uint32_t)xme_mvbits(4 * (in.omx + i - R) - pu.mvp_x));
-                wa->yt[i] = ty;
-                wa->yp[i] = ((never ? kNever : min(ty, tn) >> 16) << 5) | (uint32_t)(i & 31);
-            }
-            rs.ok = all_legal;
-            rs.cx = in.omx;
-            rs.cy = in.omy;
-            rs.px = pu.mvp_x;
-            rs.py = pu.mvp_y;
-        }
-    }
     wave_sync();
 
     const int lc = lane & ((1 << lc_log2) - 1), rg = lane >> lc_log2;
@@ -563,21 +598,22 @@ __device__ __forceinline__ void el_item(const DevParams &p, const TaskView &v, c
 #pragma unroll
     for (int d = 0; d < 2; d++) {
         const int i = 2 * lc + d;
-        lx[d] = i < lox || i > hix ? kNever : wa->xt[min(i, R2 - 1)] >> 16;
+        lx[d] = i < box.lox || i > box.hix ? kNever : wa->xt[min(i, R2 - 1)] >> 16;
     }
     const uint32_t *s_lane = v.s32 + by * v.sp + ((bx + min(2 * lc, R2 - 2)) >> 1);
 
-    uint32_t T = (uint32_t)(key0 >> 32);      // a cost that some candidate has
-    uint32_t bc = 0xFFFFFFFFu, bo = 0xFFFFFFFFu;
     int n = 0;
     const int n_bands = (nrows + band_rows - 1) / band_rows;
+    bool dense = false;
+    end_lo = row0;
+    begin_hi = row0 + nrows;
     for (int band = 0; band < n_bands; band++) {
         // bands from the centre outwards: short vectors are likelier
         const int bi = (n_bands >> 1) + ((band & 1) ? -((band + 1) >> 1) : band >> 1);
         const int row = max(row0, min(row0 + bi * band_rows + rg * K, row0 + nrows - K));
         uint32_t tk[K / 2];        // per row pair: the smallest bound of its 4 candidates
         uint32_t kmin = 0xFFFFFFFFu;
-        const bool bounds = rs.dense == 0;
+        const bool bounds = STRIPS || rs.dense == 0;
         if (!bounds) {             // every legal tile is listed
             rs.dense--;
 #pragma unroll
@@ -636,10 +672,19 @@ __device__ __forceinline__ void el_item(const DevParams &p, const TaskView &v, c
                 n += __popcll(pairs);
             }
         }
-        // noise without structure: the bounds of 9 tiles in 10 pass, and the next
-        // bands' are not worth their time
-        if (bounds && 10 * (n - n0) > 9 * ((16 * K * R) >> lc_log2))
-            rs.dense = 3;
+        // noise: most tiles pass, and costing them one by one takes longer than
+        // costing every candidate of this band and of the others
+        if (bounds && kDenseDen * (n - n0) > kDenseNum * ((16 * K * R) >> lc_log2)) {
+            if constexpr (!STRIPS) {
+                rs.dense = 3;
+            } else if (nrows >= K) {
+                n = n0;
+                end_lo = band ? row0 + ((n_bands >> 1) - (band >> 1)) * band_rows : begin_hi;
+                begin_hi = band ? min(begin_hi, row0 + ((n_bands >> 1) + ((band + 1) >> 1)) * band_rows) : begin_hi;
+                dense = true;
+                break;
+            }
+        }
         wave_sync();
         while (n >= 64) {
             n -= 64;
@@ -649,15 +694,155 @@ __device__ __forceinline__ void el_item(const DevParams &p, const TaskView &v, c
     }
     if (n > 0)
         I.template cost_tiles<false>(0, n, bc, bo);
-    const uint32_t wc = wave_min(bc);
-    const uint32_t wo = wave_min(bc == wc ? bo : 0xFFFFFFFFu);
-    const uint64_t kbest = xme_key(wc, wo);
-    if (lane == 0 && wc != 0xFFFFFFFFu && kbest < key0)
-        atomicMin(reinterpret_cast<unsigned long long *>(best + inst_id), (unsigned long long)kbest);
+    return dense;
 }
 
-// K rows per lane for PUs up to 16 x 16, KM for the larger ones.
-template <int K, int KM>
+typedef const __attribute__((address_space(3))) uint32_t *lds_dwords;
+
+// SADs of 4 columns x KD candidate rows over a strip of ND dwords x `rows` PU
+// rows (a multiple of 4; 4 ND * rows * 255 < 2^16).  The last KD window rows
+// are kept realigned, so each is read once; the next window and PU rows are in
+// flight, the last reads passing the strip by a row (inside the task's LDS).
+template <int KD, int ND>
+__device__ __forceinline__ void dense_strip(lds_dwords w, int pd, uint32_t shift, lds_dwords c, int cpd, int rows,
+                                            uint64_t (&a)[KD])
+{
+    uint64_t ring[KD][ND];
+    uint32_t raw[ND + 2], cur[2][ND];
+    auto load_c = [&](int j) {
+        asm volatile("" : "+v"(c));
+#pragma unroll
+        for (int i = 0; i < ND; i++)
+            cur[j & 1][i] = c[i];
+        c += cpd;
+    };
+    auto load = [&]() {
+        asm volatile("" : "+v"(w));        // one running address, not one per row
+#pragma unroll
+        for (int i = 0; i < ND + 2; i++)
+            raw[i] = w[i];
+        w += pd;
+    };
+    auto realign = [&](uint64_t (&d)[ND]) {
+        uint32_t al[ND + 1];
+#pragma unroll
+        for (int i = 0; i <= ND; i++)
+            al[i] = __builtin_amdgcn_alignbyte(raw[i + 1], raw[i], shift);
+#pragma unroll
+        for (int i = 0; i < ND; i++)
+            d[i] = ((uint64_t)al[i + 1] << 32) | al[i];
+    };
+    load();
+    load_c(0);
+#pragma unroll
+    for (int r = 0; r < KD - 1; r++) {
+        realign(ring[r]);
+        load();
+    }
+    for (int y = 0; y < rows; y += 8) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if (j == 4 && y + 4 >= rows)
+                break;
+            realign(ring[(j + KD - 1) % KD]);
+            load();
+            load_c(j + 1);
+#pragma unroll
+            for (int i = 0; i < ND; i++)
+#pragma unroll
+                for (int k = 0; k < KD; k++)
+                    a[k] = __builtin_amdgcn_qsad_pk_u16_u8(ring[(j + k) % KD][i], cur[j & 1][i], a[k]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+// Every candidate of rows [lo, hi) of an item, whose rows begin at row0 and are
+// at least KD, R >= 2: a lane owns 4 columns x KD rows.  Lanes past the last
+// column or row repeat others.  SMALL: PUs of at most 256 pixels, whose SADs
+// the u16 sums hold; the others' sides are multiples of 8.
+template <int KD, bool SMALL>
+__device__ __forceinline__ void dense_rows(const DevParams &p, const TaskView &v, const DevPu &pu, const DevInst &in,
+                                           bool all_legal, int row0, int lo, int hi, int lc_log2,
+                                           const WaveArea *__restrict__ wa, uint32_t &bc, uint32_t &bo)
+{
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int R = p.R, qc_log2 = lc_log2 - 1;
+    const int col = min(4 * (lane & ((1 << qc_log2) - 1)), 2 * R - 4), g = lane >> qc_log2;
+    const int x0 = pu.x + in.omx - R - v.wx0 + col, by = pu.y + in.omy - R - v.wy0;
+    const uint32_t shift = (uint32_t)x0 & 3u;
+    const lds_dwords cpu32 = (lds_dwords)(v.c32 + (pu.y - v.cy0) * v.cpd + ((pu.x - v.cx0) >> 2));
+    for (int base = lo; base < hi; base += (64 >> qc_log2) * KD) {
+        const int row = max(row0, min(base + g * KD, hi - KD));
+        const lds_dwords w = (lds_dwords)(v.w32 + (by + row) * v.pd + (x0 >> 2));
+        uint32_t sad[KD][4];
+        uint64_t a[KD];
+        auto unpack = [&]() {
+#pragma unroll
+            for (int k = 0; k < KD; k++) {
+                sad[k][0] += (uint32_t)a[k] & 0xFFFFu;
+                sad[k][1] += (uint32_t)a[k] >> 16;
+                sad[k][2] += (uint32_t)(a[k] >> 32) & 0xFFFFu;
+                sad[k][3] += (uint32_t)(a[k] >> 48);
+                a[k] = 0;
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < KD; k++) {
+            a[k] = 0;
+            sad[k][0] = sad[k][1] = sad[k][2] = sad[k][3] = 0;
+        }
+        if constexpr (SMALL) {
+            if (pu.w & 7)
+                for (int x = 0; x < pu.w >> 2; x++)
+                    dense_strip<KD, 1>(w + x, v.pd, shift, cpu32 + x, v.cpd, pu.h, a);
+            else
+                for (int x = 0; x < pu.w >> 2; x += 2)
+                    dense_strip<KD, 2>(w + x, v.pd, shift, cpu32 + x, v.cpd, pu.h, a);
+            unpack();
+        } else {
+            for (int x = 0; x < pu.w >> 2; x += 2)
+                for (int y = 0; y < pu.h; y += 32) {
+                    dense_strip<KD, 2>(w + y * v.pd + x, v.pd, shift, cpu32 + y * v.cpd + x, v.cpd, min(32, pu.h - y), a);
+                    unpack();
+                }
+        }
+        uint32_t key = 0xFFFFFFFFu;
+#pragma unroll
+        for (int k = 0; k < KD; k++) {
+            const uint32_t ty = wa->yt[row + k];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                sad[k][c] = ((sad[k][c] + ((wa->xt[col + c] + ty) >> 16)) << 5) | (uint32_t)(4 * k + c);
+        }
+        if (all_legal) {
+#pragma unroll
+            for (int k = 0; k < KD; k++)
+                key = min(key, min(min(sad[k][0], sad[k][1]), min(sad[k][2], sad[k][3])));
+        } else {
+            const MvWindow mw = xme_mv_window(p, pu.x, pu.y, pu.w, pu.h);
+#pragma unroll
+            for (int k = 0; k < KD; k++)
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    if (xme_mv_legal(mw, in.omx + col + c - R, in.omy + row + k - R))
+                        key = min(key, sad[k][c]);
+        }
+        const uint32_t cost = key >> 5;
+        const uint32_t order =
+            XME_ORDER_RASTER + (uint32_t)((row + (int)((key >> 2) & 7)) * 2 * R + col + (int)(key & 3));
+        if (key != 0xFFFFFFFFu && (cost < bc || (cost == bc && order < bo))) {
+            bc = cost;
+            bo = order;
+        }
+    }
+}
+
+// K rows per lane for PUs up to 16 x 16, KM for the larger ones.  STRIPS: see
+// kDenseNum; a template parameter, since as a branch in the loop over bands it
+// cost every picture 2 %.
+template <int K, int KM, bool STRIPS>
 __global__ void __launch_bounds__(1024) elim_kernel(DevParams p, const FrameDesc *__restrict__ desc,
                                                     const DevInst *__restrict__ inst,
                                                     const FsTask *__restrict__ tasks, int n_tasks,
@@ -668,6 +853,8 @@ __global__ void __launch_bounds__(1024) elim_kernel(DevParams p, const FrameDesc
     __shared__ int s_task;
     __shared__ int s_item;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    WaveState rs;
+    rs.dense = rs.run = 0;
     for (;;) {
         if (threadIdx.x == 0)
             s_task = (int)atomicAdd(&counters[0], 1u);
@@ -699,9 +886,8 @@ __global__ void __launch_bounds__(1024) elim_kernel(DevParams p, const FrameDesc
         build_sums(t, l32, v.pd, s32, v.sp);
         __syncthreads();
         WaveArea *wa = reinterpret_cast<WaveArea *>(a32) + wave;
-        WaveState rs;
         rs.ok = false;
-        rs.cx = rs.cy = rs.px = rs.py = rs.dense = 0;
+        rs.cx = rs.cy = rs.px = rs.py = 0;
         for (;;) {
             int it = 0;
             if ((threadIdx.x & 63) == 0)
@@ -723,27 +909,57 @@ __global__ void __launch_bounds__(1024) elim_kernel(DevParams p, const FrameDesc
             pu.h = item.h;
             pu.mvp_x = item.mvp_x;
             pu.mvp_y = item.mvp_y;
+            const Box box = rate_terms(p, pu, in, wa, rs);
+            uint32_t bc = 0xFFFFFFFFu, bo = 0xFFFFFFFFu;
+            // rows still to search when it leaves some: before and after its bands
+            int from[2] = { item.row0, 0 }, to[2] = { item.row0 + item.nrows, 0 };
+            if (STRIPS && rs.dense > 0 && item.nrows >= (pu.w > 16 || pu.h > 16 ? KM : K)) {
+                rs.dense--;
+            } else {
+                bool dense = false;
 #define XME_EL(NXX, NYY, ONE)                                                                                  \
-    el_item<ONE ? K : KM, NXX, NYY, ONE>(p, v, pu, in, item.inst, item.row0, item.nrows, lc_log2, key0, best, wa, rs)
-            switch (pu.w * 64 + pu.h) {
-            case 8 * 64 + 8: XME_EL(2, 2, true); break;
-            case 16 * 64 + 16: XME_EL(4, 4, true); break;
-            case 16 * 64 + 8: XME_EL(4, 2, true); break;
-            case 8 * 64 + 16: XME_EL(2, 4, true); break;
-            case 16 * 64 + 12: XME_EL(4, 3, true); break;
-            case 12 * 64 + 16: XME_EL(3, 4, true); break;
-            case 16 * 64 + 4: XME_EL(4, 1, true); break;
-            case 4 * 64 + 16: XME_EL(1, 4, true); break;
-            case 8 * 64 + 4: XME_EL(2, 1, true); break;
-            case 4 * 64 + 8: XME_EL(1, 2, true); break;
-            case 4 * 64 + 4: XME_EL(1, 1, true); break;
-            case 32 * 64 + 8:
-            case 32 * 64 + 24: XME_EL(4, 2, false); break;
-            case 8 * 64 + 32:
-            case 24 * 64 + 32: XME_EL(2, 4, false); break;
-            default: XME_EL(4, 4, false); break;       // multiples of 16 on both sides
-            }
+    dense = el_item<ONE ? K : KM, NXX, NYY, ONE, STRIPS>(p, v, pu, in, box, item.row0, item.nrows, lc_log2,    \
+                                                         (uint32_t)(key0 >> 32), wa, rs, bc, bo, to[0], from[1])
+                switch (pu.w * 64 + pu.h) {
+                case 8 * 64 + 8: XME_EL(2, 2, true); break;
+                case 16 * 64 + 16: XME_EL(4, 4, true); break;
+                case 16 * 64 + 8: XME_EL(4, 2, true); break;
+                case 8 * 64 + 16: XME_EL(2, 4, true); break;
+                case 16 * 64 + 12: XME_EL(4, 3, true); break;
+                case 12 * 64 + 16: XME_EL(3, 4, true); break;
+                case 16 * 64 + 4: XME_EL(4, 1, true); break;
+                case 4 * 64 + 16: XME_EL(1, 4, true); break;
+                case 8 * 64 + 4: XME_EL(2, 1, true); break;
+                case 4 * 64 + 8: XME_EL(1, 2, true); break;
+                case 4 * 64 + 4: XME_EL(1, 1, true); break;
+                case 32 * 64 + 8:
+                case 32 * 64 + 24: XME_EL(4, 2, false); break;
+                case 8 * 64 + 32:
+                case 24 * 64 + 32: XME_EL(2, 4, false); break;
+                default: XME_EL(4, 4, false); break;       // multiples of 16 on both sides
+                }
 #undef XME_EL
+                to[1] = item.row0 + item.nrows;
+                if (STRIPS)
+                    rs.dense = rs.run = dense ? min(4 * rs.run + 3, kDenseRun) : 0;
+            }
+            if constexpr (STRIPS) {
+                for (int k = 0; k < 2; k++) {
+                    if (from[k] >= to[k])
+                        continue;
+                    if (pu.w * pu.h > 256)
+                        dense_rows<KM / 2, false>(p, v, pu, in, box.all_legal, item.row0, from[k], to[k], lc_log2, wa, bc, bo);
+                    else if (KM < K && (pu.w > 16 || pu.h > 16))
+                        dense_rows<KM / 2, true>(p, v, pu, in, box.all_legal, item.row0, from[k], to[k], lc_log2, wa, bc, bo);
+                    else
+                        dense_rows<K / 2, true>(p, v, pu, in, box.all_legal, item.row0, from[k], to[k], lc_log2, wa, bc, bo);
+                }
+            }
+            const uint32_t wc = wave_min(bc);
+            const uint32_t wo = wave_min(bc == wc ? bo : 0xFFFFFFFFu);
+            const uint64_t kbest = xme_key(wc, wo);
+            if ((threadIdx.x & 63) == 0 && wc != 0xFFFFFFFFu && kbest < key0)
+                atomicMin(reinterpret_cast<unsigned long long *>(best + item.inst), (unsigned long long)kbest);
         }
         __syncthreads();   // LDS is reused by the next task
     }
@@ -799,11 +1015,26 @@ __global__ void __launch_bounds__(256) cost_map_kernel(DevParams p, const FrameD
     }
 }
 
-const void *kernel_ptr(int K, int KM)
+const void *const kKernels[5] = {
+    reinterpret_cast<const void *>(&elim_kernel<4, 4, false>),
+    reinterpret_cast<const void *>(&elim_kernel<16, 8, false>),
+    reinterpret_cast<const void *>(&elim_kernel<16, 8, true>),
+    reinterpret_cast<const void *>(&elim_kernel<16, 16, false>),
+    reinterpret_cast<const void *>(&elim_kernel<16, 16, true>),
+};
+
+// Whether noise is costed in strips rather than as listed tiles: with 16 rows
+// per lane (at 4, R < 24, elimination is the quicker one on noise too) and
+// where 3/4 of dense_rows' lanes have a candidate of their own, or 9/16 for odd
+// R, whose tiles cost more.  1080p noise, mixed PUs, listed and in strips: R =
+// 34 220 and 267 us, 48 330 and 333, 52 409 and 366, 49 495 and 403, 64 488 and
+// 391.
+bool el_strips(int R)
 {
-    return K == 4    ? reinterpret_cast<const void *>(&elim_kernel<4, 4>)
-           : KM == 8 ? reinterpret_cast<const void *>(&elim_kernel<16, 8>)
-                     : reinterpret_cast<const void *>(&elim_kernel<16, 16>);
+    if (R < 24)
+        return false;
+    const int lc = xme_el_lc_log2(R), band = (64 >> lc) * 16;
+    return 64 * R * R > (R & 1 ? 9 : 12) * (2 << lc) * ((2 * R + band - 1) / band * band);
 }
 
 } // namespace
@@ -832,7 +1063,7 @@ int xme_el_prepare(void)
     static std::once_flag once;
     static hipError_t err = hipSuccess;
     std::call_once(once, [] {
-        for (const void *k : { kernel_ptr(4, 4), kernel_ptr(16, 8), kernel_ptr(16, 16) })
+        for (const void *k : kKernels)
             if (err == hipSuccess)
                 err = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, xme_fs_max_lds());
     });
@@ -843,7 +1074,9 @@ int xme_el_prepare(void)
 
 const void *xme_el_kernel_ptr(int R, bool few_tasks)
 {
-    return kernel_ptr(xme_el_rows(R, few_tasks, 4, 4), xme_el_rows(R, few_tasks, 64, 64));
+    if (xme_el_rows(R, few_tasks, 4, 4) == 4)
+        return kKernels[0];
+    return kKernels[(xme_el_rows(R, few_tasks, 64, 64) == 8 ? 1 : 3) + (el_strips(R) ? 1 : 0)];
 }
 
 int xme_launch_elim(const DevParams &p, const FrameDesc *d_desc, const DevInst *d_inst, const FsTask *d_tasks,
