@@ -1157,6 +1157,9 @@ def main():
     search_ms, job_ms, _ = plan.time(dcur, d_refs, stream.h, 5)
     exhaustive_equiv = n_absdiff / (search_ms * 1e-3) / 1e12
     log(f"search kernel {search_ms:.3f} ms, the work of {exhaustive_equiv:.1f} T absdiff/s by exhaustion")
+    # what the elimination cannot do without at the VALU's peak (16 lanes a SIMD
+    # cycle): a lane-operation per 32 pixels of every legal candidate
+    bounds_ms = n_absdiff / 32 / (VALU_PEAK_TCYCLES * 1e12 * 16) * 1e3 if R <= 64 else None
 
     # plain path: one launch per PU shape, no persistent queue, no graph
     log("timing the plain path")
@@ -1224,8 +1227,6 @@ def main():
             "integer_candidates_per_step": int(n_cand),
             "exhaustive_absdiffs_per_step": int(n_absdiff),
             "lambda_factor": lam,
-            "tiles_K_LC": {str(k): v for k, v in tiles.items()},
-            "tiles_tuned_in_run": tuned_now,
         },
         "roofline": {
             "bound": "valu",
@@ -1233,6 +1234,11 @@ def main():
             "peak": VALU_PEAK_TCYCLES,
             "unit": "T SIMD cycles/s with a vector instruction (SQ_ACTIVE_INST_VALU, measured in this run)",
             "frac": achieved / VALU_PEAK_TCYCLES if achieved else None,
+            "frac_is": "issue utilisation: cycles with any vector instruction, needed or not",
+            "bounds_ms": bounds_ms,
+            "bounds_frac": bounds_ms / search_ms if bounds_ms else None,
+            "bounds_are": "needed work at the VALU's peak: the bounds of all legal candidates, without the exact costs "
+                          "of those that pass",
             "exhaustive_equivalent_tabsdiff_per_s": exhaustive_equiv,
             "traffic": traffic,
             "traffic_unit": "HBM bytes per search step, measured in this run: rocprofv3 --pmc FETCH_SIZE and "
@@ -1242,7 +1248,9 @@ def main():
             "kernel": "integer full search by elimination, elim_kernel (range > 64: fs_kernel), persistent",
             "kernel_ms": search_ms,
         },
-        "plain": {"value": plain_value, "ms_per_step": plain_ms, "results_equal": plain_equal},
+        "plain": {"value": plain_value, "ms_per_step": plain_ms, "results_equal": plain_equal,
+                  # the exhaustive kernels' tile shapes; a batched search of ranges up to 64 has none
+                  "tiles_K_LC": {str(k): v for k, v in tiles.items()}, "tiles_tuned_in_run": tuned_now},
         "speedup_vs_plain": value / plain_value,
         "latency_ms": {"p50": float(np.percentile(lat, 50)), "p99": float(np.percentile(lat, 99)),
                        "mean": float(lat.mean())},
