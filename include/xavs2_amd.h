@@ -267,7 +267,10 @@ int xme_plan_search_count(const xme_plan *plan, int64_t *n_points, int64_t *n_ab
 int xme_plan_set_umh_context(xme_plan *plan, const xme_umh_ctx *ctx, void *stream);
 /* Caps the workgroups of the batched plan's persistent search launch (0 =
  * as many as the device holds at once), so that searches of concurrent
- * frames share the compute units instead of queueing behind each other. */
+ * frames share the compute units instead of queueing behind each other.  Give
+ * a share of xme_plan_workgroups' device_fill rather than a fixed number: a
+ * workgroup has 256 threads in the exhaustive search (ranges over 64), and 512
+ * or 1024 in the other, where it may hold a whole compute unit's LDS. */
 int xme_plan_set_max_workgroups(xme_plan *plan, int max_workgroups);
 int xme_plan_workgroups(const xme_plan *plan, int *workgroups, int *device_fill);
 /* Splits the batched plan's search into launches of at most this many
